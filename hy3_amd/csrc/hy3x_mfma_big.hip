@@ -144,8 +144,7 @@ __device__ __forceinline__ void big_step(State<GATEUP, NTT> &st, int s) {
 
   const u4_t *as = &a_ring[kb & 1][0];
   const u4_t *xs = &bx[s & 1][0];
-  const uint32_t sel =
-      0x0C000C00u | ((uint32_t)(2 * (g >> 1) + 1) << 16) | (uint32_t)(2 * (g >> 1));
+  const uint32_t sel = bytes_sel(g >> 1), msel = bytes_sel(g & 1);
   const int gch = 8 * (g >> 1) + 2 * (g & 1);
   const f4_t zero4 = {0.f, 0.f, 0.f, 0.f};
   u4_t pv[RG][NMAT];
@@ -163,13 +162,9 @@ __device__ __forceinline__ void big_step(State<GATEUP, NTT> &st, int s) {
 #pragma unroll
     for (int m = 0; m < NMAT; m++) {
       const Scales6 s6 = unpack_scales(st.hdr[rg][m]);
-      const h2_t sc = bytes_h2(h ? s6.sc[1] : s6.sc[0], sel);
-      const h2_t mul = sc * (h2_t){(_Float16)1.0f, (_Float16)0.0625f};
-      const h2_t add = sc * (h2_t){(_Float16)-1024.0f, (_Float16)-64.0f};
-      const h2_t ml = {mul[0], mul[0]}, al = {add[0], add[0]};
-      const h2_t mh = {mul[1], mul[1]}, ah = {add[1], add[1]};
-      dequant_run(pv[rg][m].xy, ml, al, mh, ah, wf[rg][m][0], wf[rg][m][2]);
-      dequant_run(pv[rg][m].zw, ml, al, mh, ah, wf[rg][m][1], wf[rg][m][3]);
+      const PairScale ps = pair_scale(h ? s6.sc[1] : s6.sc[0], sel);
+      dequant_run(pv[rg][m].xy, ps, wf[rg][m][0], wf[rg][m][2]);
+      dequant_run(pv[rg][m].zw, ps, wf[rg][m][1], wf[rg][m][3]);
     }
   // k run outer, token groups inner: an MFMA's accumulator was last written
   // 2 NTT MFMAs earlier, so the chains do not wait on each other
@@ -194,10 +189,9 @@ __device__ __forceinline__ void big_step(State<GATEUP, NTT> &st, int s) {
 #pragma unroll
       for (int m = 0; m < NMAT; m++) {
         const u4_t hd = st.hdr[rg][m];
-        const float d = fp16_quirk(hd.x & 0xffffu), dmin = fp16_quirk(hd.x >> 16);
+        const float d = fp16_quirk(hd.x & 0xffffu);
         const Scales6 s6 = unpack_scales(hd);
-        const uint32_t mw = (g >> 1) ? s6.mn[1] : s6.mn[0];
-        const h8_t mo = mins_operand(dmin, (g & 1) ? (mw >> 16) : mw);
+        const h8_t mo = mins_operand(hd.x, (g >> 1) ? s6.mn[1] : s6.mn[0], msel);
 #pragma unroll
         for (int t = 0; t < NTT; t++) {
           const h8_t sv = __builtin_bit_cast(

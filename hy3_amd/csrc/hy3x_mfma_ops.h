@@ -42,12 +42,28 @@ __device__ __forceinline__ Scales6 unpack_scales(const u4_t &h) {
   return r;
 }
 
-// fp16 pair of the two bytes of w that `sel` (a v_perm selector placing them
-// in bytes 0 and 2, zeros in 1 and 3) picks, values <= 63: the bytes go into
-// the mantissa of 1024.0, then 1024 is subtracted (both steps exact).
+// The two bytes of w that `sel` picks (a v_perm selector: their indices in its
+// bytes 0 and 2, 4 in bytes 1 and 3) as the fp16 pair 1024 + byte: each byte
+// goes into the mantissa of 1024.0.
 __device__ __forceinline__ h2_t bytes_h2(uint32_t w, uint32_t sel) {
-  const uint32_t v = __builtin_amdgcn_perm(w, w, sel) | 0x64006400u;
-  return as_h2(v) + (h2_t){(_Float16)-1024.0f, (_Float16)-1024.0f};
+  return as_h2(__builtin_amdgcn_perm(0x64646464u, w, sel));
+}
+// The selector of bytes 2 i and 2 i + 1.
+__device__ __forceinline__ uint32_t bytes_sel(int i) {
+  return 0x04000400u | (uint32_t)(2 * i + 1) << 16 | (uint32_t)(2 * i);
+}
+
+// The scales of a lane's sub-block pair (a low- and a high-nibble sub-block) as
+// the operands of dequant_run: (sc_lo, sc_hi / 16) and -(1024 sc_lo, 64 sc_hi).
+struct PairScale {
+  h2_t mul, add;
+};
+__device__ __forceinline__ PairScale pair_scale(uint32_t scw, uint32_t sel) {
+  const h2_t sc = bytes_h2(scw, sel) - (h2_t){(_Float16)1024.0f, (_Float16)1024.0f};
+  PairScale r;
+  r.mul = sc * (h2_t){(_Float16)1.0f, (_Float16)0.0625f};
+  r.add = sc * (h2_t){(_Float16)-1024.0f, (_Float16)-64.0f};
+  return r;
 }
 
 // Weight operands of one 8-byte run of qs: the low nibbles (sub-block scale
@@ -56,8 +72,10 @@ __device__ __forceinline__ h2_t bytes_h2(uint32_t w, uint32_t sel) {
 // High, left in place: 0x6400 | 16q = 1024 + 16q, times sc_hi/16, minus
 // 64 sc_hi. Each is one fused multiply-add whose exact result is
 // representable, so it is exact.
-__device__ __forceinline__ void dequant_run(u2_t q, h2_t ml, h2_t al, h2_t mh, h2_t ah,
-                                            h8_t &w_lo, h8_t &w_hi) {
+__device__ __forceinline__ void dequant_run(u2_t q, const PairScale &ps, h8_t &w_lo,
+                                            h8_t &w_hi) {
+  const h2_t ml = {ps.mul[0], ps.mul[0]}, al = {ps.add[0], ps.add[0]};
+  const h2_t mh = {ps.mul[1], ps.mul[1]}, ah = {ps.add[1], ps.add[1]};
   const uint32_t mag = 0x64006400u, m_lo = 0x000F000Fu, m_hi = 0x00F000F0u;
   const uint32_t x8 = q.x >> 8, y8 = q.y >> 8;
   u4_t lo, hi;
@@ -73,16 +91,26 @@ __device__ __forceinline__ void dequant_run(u2_t q, h2_t ml, h2_t al, h2_t mh, h
   w_hi = __builtin_bit_cast(h8_t, hi);
 }
 
-// -dmin * m_j for sub-blocks j = 2g and 2g+1 of this lane's row, each split
-// exactly into two fp16 parts (dmin: 11 significant bits, m: 6, so the
-// product is exact in fp32 and hi + lo carries it to 22 bits), laid out for
-// the mins MFMA: k = 4j' + c, c = (hi, hi, lo, lo) against the staged
-// activation sums (Sh, Sl, Sh, Sl): the four cross products of the two splits.
-__device__ __forceinline__ h8_t mins_operand(float dmin, uint32_t m2) {
-  const float v0 = -dmin * (float)(m2 & 0xFFu), v1 = -dmin * (float)((m2 >> 8) & 0xFFu);
-  const _Float16 h0 = (_Float16)v0, h1 = (_Float16)v1;
-  const _Float16 l0 = (_Float16)(v0 - (float)h0), l1 = (_Float16)(v1 - (float)h1);
-  return (h8_t){h0, h0, l0, l0, h1, h1, l1, l1};
+// The mins operand of a row-block (header hd) for the lane's sub-blocks j = 2g
+// and 2g + 1 (their mins in the bytes of mw that sel picks): -dmin * m_j, each
+// split exactly into two fp16 parts hi + lo (dmin: 11 significant bits, m: 6;
+// the product's rounding error is one fused multiply-add away), against the
+// staged activation sums (Sh, Sl, Sh, Sl): the four cross products of the two
+// splits fill the MFMA's k slots. dmin is used as the half it is stored as:
+// hy3.c's decode (fp16_quirk) reads a half with exponent 0 as 2^-15 (1 + mant /
+// 1024), half of the half with exponent 1 and the same mantissa, so there m / 2
+// (exact) meets that one. In packed fp16 this takes nine vector instructions;
+// through fp32 conversions it took 28, of about 260 per wave and column.
+__device__ __forceinline__ h8_t mins_operand(uint32_t hx, uint32_t mw, uint32_t sel) {
+  const bool z = (hx & 0x7C000000u) == 0u;
+  const _Float16 dmin = __builtin_bit_cast(_Float16, (uint16_t)((hx >> 16) | (z ? 0x0400u : 0u)));
+  const _Float16 f1 = z ? (_Float16)0.5f : (_Float16)1.0f;
+  const _Float16 f0 = z ? (_Float16)-512.0f : (_Float16)-1024.0f;
+  const h2_t nd = {-dmin, -dmin};
+  const h2_t m = __builtin_elementwise_fma(bytes_h2(mw, sel), (h2_t){f1, f1}, (h2_t){f0, f0});
+  const h2_t hi = m * nd;
+  const h2_t lo = __builtin_elementwise_fma(m, nd, -hi);
+  return (h8_t){hi[0], hi[1], hi[0], hi[1], lo[0], lo[1], lo[0], lo[1]};
 }
 
 // Launch order -> work item, so that consecutive work items run on one XCD

@@ -118,8 +118,11 @@ __device__ __forceinline__ void load_group_x(const __half *staged, int g, uint32
   }
 }
 
-// Sub-block sums of one fp16 row of n32 * 32 values, as (Sh, Sl, Sh, Sl) with
-// Sh = fp16(sum), Sl = fp16(sum - Sh). One lane per sub-block.
+// Sub-block sums of one fp16 row of n32 * 32 values (n32 even), split into
+// fp16 parts Sh = fp16(sum), Sl = fp16(sum - Sh). Sub-blocks 2g and 2g + 1 share
+// 16 bytes, (Sh, Sh), (Sl, Sl), (Sh, Sh), (Sl, Sl): an MFMA lane's k slots of
+// the mins product (mins_operand). One lane per sub-block; each lane of a pair
+// writes half of its 16 bytes.
 __device__ __forceinline__ void row_subsums(const __half *__restrict__ row, int n32,
                                             __half *__restrict__ dst) {
   for (int j = threadIdx.x; j < n32; j += blockDim.x) {
@@ -138,9 +141,13 @@ __device__ __forceinline__ void row_subsums(const __half *__restrict__ row, int 
     }
     const _Float16 hi = (_Float16)sum;
     const _Float16 lo = (_Float16)(sum - (float)hi);
-    const h2_t r = {hi, lo};
-    *reinterpret_cast<h2_t *>(dst + 4 * j) = r;
-    *reinterpret_cast<h2_t *>(dst + 4 * j + 2) = r;
+    const uint32_t own = __builtin_bit_cast(uint32_t, (h2_t){hi, lo});
+    const uint32_t oth = (uint32_t)__shfl_xor((int)own, 1, 64);
+    const uint32_t e = j & 1 ? oth : own, o = j & 1 ? own : oth;  // even, odd sub-block
+    uint2 r;
+    r.x = (e & 0xffffu) | (o << 16);
+    r.y = (e >> 16) | (o & 0xffff0000u);
+    *reinterpret_cast<uint2 *>(dst + 4 * j) = r;
   }
 }
 
