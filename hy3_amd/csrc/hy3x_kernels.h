@@ -7,9 +7,9 @@ namespace hy3x {
 __global__ void k_router_logits(const float *x, const float *xadd, const float *norm_w,
                                 const float *router,
                                 const float *bias, int has_bias, float *logits, float *sig,
-                                float *score, __half *s16, float *s32,
-                                unsigned long long *trace, int T, uint32_t *bits, int wt,
-                                const float *r_in);
+                                float *score, __half *s16, float *s32, __half *s16m,
+                                __half *ssum, unsigned long long *trace, int T,
+                                uint32_t *bits, int wt, const float *r_in);
 __global__ void k_rmsnorm(const float *x, const float *xadd, const float *norm_w, __half *s16,
                           float *s32,
                           __half *s16m, __half *ssum, int T, uint32_t *bits, int wt,
@@ -73,6 +73,17 @@ __global__ void k_dispatch_list(const uint8_t *ranks, int T, int K, int NT, cons
                                 int wt, int32_t *list, int4 *tiles,
                                 int32_t *n_tiles, int max_tiles, int32_t *counts_out,
                                 unsigned long long *stats);
+// Up to this many tokens one block routes every token and makes the dispatch
+// lists (k_route_small), in one launch where top-K, staging and dispatch were
+// three: 2 / 3 / 4 / 8 tokens 73.4 / 99.5 / 108.0 / 155.9 -> 64.4 / 90.0 / 98.3 /
+// 145.9 us per forward. It ends where the router stops running one wave per
+// (expert, token) and one wave per token still fits one block; the T > 8 router
+// stages s in k_rmsnorm and its dispatch alone takes about 4 us.
+constexpr int ROUTE_SMALL_T = 8;
+__global__ void k_route_small(const float *logits, const float *bias, int has_bias, int K,
+                              float scale, int T, int NT, int32_t *ids, float *wpre, float *wout,
+                              int32_t *list, int4 *tiles, int32_t *n_tiles, int max_tiles,
+                              int32_t *counts_out, unsigned long long *stats);
 template <int NT>
 __global__ void k_gateup_gemv(const uint8_t *wq, const __half *s16, const int32_t *list,
                               const int4 *tiles, const int32_t *n_tiles, int T, int K,
@@ -159,7 +170,6 @@ extern template __global__ void k_moe_big<false>(const uint8_t *, const uint8_t 
                                                  const int32_t *, const int4 *, const int32_t *,
                                                  int, int, __half *, float *);
 }  // namespace mfma_big
-__global__ void k_stage_mfma(const float *s32, __half *s16m, __half *ssum);
 __global__ void k_hsums(const __half *h16m, __half *hsum);
 
 __global__ void k_synth_q4k(uint8_t *dst, int64_t nblocks, uint64_t seed, uint32_t layer,

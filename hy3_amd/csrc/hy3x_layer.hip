@@ -502,11 +502,15 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
         break;
       }
       // the routing kernels also clear (first kernel) and fill (top-K) the
-      // dispatch bitmaps; for T > 8 the RMSNorm kernel stages the MFMA operand
+      // dispatch bitmaps, or make the lists themselves (k_route_small); the
+      // first kernel stages the MFMA operand
       if (T <= kSmallRouterT) {
+        const bool mf = c.mode == Mode::MFMA;
         k_router_logits<<<dim3(E, T), 256, 0, st>>>(x, c.xadd, L->norm_w, L->router, L->bias,
                                                     L->has_bias, S.logits, S.sig, S.score,
-                                                    S.s16, S.s32, L->trace[0], T, S.bits,
+                                                    S.s16, S.s32, mf ? S.s16m : nullptr,
+                                                    S.ssum, L->trace[0], T,
+                                                    T <= ROUTE_SMALL_T ? nullptr : S.bits,
                                                     S.wt, c.r_in);
       } else {
         const bool mf = c.mode == Mode::MFMA;
@@ -529,7 +533,11 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
           HY3X_LAUNCH_ROUTER(XXL);
 #undef HY3X_LAUNCH_ROUTER
       }
-      {
+      if (T <= ROUTE_SMALL_T) {
+        k_route_small<<<1, 64 * ROUTE_SMALL_T, 0, st>>>(
+            S.logits, L->bias, L->has_bias, K, c.scale, T, c.nt, S.ids, S.wpre, S.w, S.list,
+            S.tiles, S.n_tiles, mt, S.counts, L->stats);
+      } else {
         // one wave per token; up to 256 tokens one wave per block, so that
         // few tokens still spread over many CUs
         const int wpb = T <= 256 ? 1 : 4;
@@ -539,9 +547,7 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
       }
       break;
     case HY3X_STAGE_DISPATCH:
-      if (c.mode == Mode::MFMA && T <= kSmallRouterT)
-        k_stage_mfma<<<T, 256, 0, st>>>(S.s32, S.s16m, S.ssum);
-      if (c.mode != Mode::DECODE) {
+      if (c.mode != Mode::DECODE && T > ROUTE_SMALL_T) {
         k_dispatch_list<<<E + 1, 256, 0, st>>>(S.ranks, T, K, c.nt, S.bits, S.wt,
                                                S.list, S.tiles, S.n_tiles, mt, S.counts,
                                                L->stats);

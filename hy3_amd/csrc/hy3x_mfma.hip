@@ -629,18 +629,6 @@ template __global__ void k_moe_mfma<false>(const uint8_t *, const uint8_t *, con
 
 #ifndef HY3X_MFMA_WIDE
 
-// fp16 copy of s in the MFMA run order (perm8) for the gate/up activations,
-// and its 128 sub-block sums.
-__global__ __launch_bounds__(256) void k_stage_mfma(const float *__restrict__ s32,
-                                                    __half *__restrict__ s16m,
-                                                    __half *__restrict__ ssum) {
-  const int t = blockIdx.x;
-  for (int j = threadIdx.x; j < D; j += 256)
-    s16m[(size_t)t * D + perm8(j)] = __float2half(s32[(size_t)t * D + j]);
-  __syncthreads();
-  row_subsums(s16m + (size_t)t * D, D / 32, ssum + (size_t)t * (D / 32) * 4);
-}
-
 // The 48 sub-block sums of every h row (down-GEMM mins operand); one wave per slot.
 __global__ __launch_bounds__(64) void k_hsums(const __half *__restrict__ h16m,
                                               __half *__restrict__ hsum) {

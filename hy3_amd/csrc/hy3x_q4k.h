@@ -118,36 +118,51 @@ __device__ __forceinline__ void load_group_x(const __half *staged, int g, uint32
   }
 }
 
-// Sub-block sums of one fp16 row of n32 * 32 values (n32 even), split into
-// fp16 parts Sh = fp16(sum), Sl = fp16(sum - Sh). Sub-blocks 2g and 2g + 1 share
-// 16 bytes, (Sh, Sh), (Sl, Sl), (Sh, Sh), (Sl, Sl): an MFMA lane's k slots of
-// the mins product (mins_operand). One lane per sub-block; each lane of a pair
-// writes half of its 16 bytes.
+// The sum of sub-block j of an fp16 row into dst, split into fp16 parts Sh =
+// fp16(sum), Sl = fp16(sum - Sh). Sub-blocks 2g and 2g + 1 share 16 bytes, (Sh,
+// Sh), (Sl, Sl), (Sh, Sh), (Sl, Sl): an MFMA lane's k slots of the mins product
+// (mins_operand). Neighbouring lanes hold neighbouring sub-blocks; each lane of
+// a pair writes half of its 16 bytes.
+__device__ __forceinline__ void store_subsum(__half *__restrict__ dst, int j, float sum) {
+  const _Float16 hi = (_Float16)sum;
+  const _Float16 lo = (_Float16)(sum - (float)hi);
+  const uint32_t own = __builtin_bit_cast(uint32_t, (h2_t){hi, lo});
+  const uint32_t oth = (uint32_t)__shfl_xor((int)own, 1, 64);
+  const uint32_t e = j & 1 ? oth : own, o = j & 1 ? own : oth;  // even, odd sub-block
+  uint2 r;
+  r.x = (e & 0xffffu) | (o << 16);
+  r.y = (e >> 16) | (o & 0xffff0000u);
+  *reinterpret_cast<uint2 *>(dst + 4 * j) = r;
+}
+
+// The sum of 32 staged fp16 values (16 pairs), in their staged order.
+__device__ __forceinline__ float subsum16(const uint32_t (&w)[16]) {
+  float sum = 0.0f;
+#pragma unroll
+  for (int u = 0; u < 16; u++) {
+    const h2_t p = as_h2(w[u]);
+    sum += (float)p[0];
+    sum += (float)p[1];
+  }
+  return sum;
+}
+
+// Sub-block sums of one fp16 row of n32 * 32 values (n32 even), one lane per
+// sub-block.
 __device__ __forceinline__ void row_subsums(const __half *__restrict__ row, int n32,
                                             __half *__restrict__ dst) {
   for (int j = threadIdx.x; j < n32; j += blockDim.x) {
     const uint4 *src = reinterpret_cast<const uint4 *>(row + 32 * j);
-    float sum = 0.0f;
+    uint32_t w[16];
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       const uint4 q = src[v];
-      const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-#pragma unroll
-      for (int u = 0; u < 4; u++) {
-        const h2_t p = as_h2(w[u]);
-        sum += (float)p[0];
-        sum += (float)p[1];
-      }
+      w[4 * v] = q.x;
+      w[4 * v + 1] = q.y;
+      w[4 * v + 2] = q.z;
+      w[4 * v + 3] = q.w;
     }
-    const _Float16 hi = (_Float16)sum;
-    const _Float16 lo = (_Float16)(sum - (float)hi);
-    const uint32_t own = __builtin_bit_cast(uint32_t, (h2_t){hi, lo});
-    const uint32_t oth = (uint32_t)__shfl_xor((int)own, 1, 64);
-    const uint32_t e = j & 1 ? oth : own, o = j & 1 ? own : oth;  // even, odd sub-block
-    uint2 r;
-    r.x = (e & 0xffffu) | (o << 16);
-    r.y = (e >> 16) | (o & 0xffff0000u);
-    *reinterpret_cast<uint2 *>(dst + 4 * j) = r;
+    store_subsum(dst, j, subsum16(w));
   }
 }
 

@@ -34,11 +34,12 @@ __global__ __launch_bounds__(256) void k_router_logits(
     const float *__restrict__ x, const float *__restrict__ xadd, const float *__restrict__ norm_w,
     const float *__restrict__ router, const float *__restrict__ bias, int has_bias,
     float *__restrict__ logits, float *__restrict__ sig, float *__restrict__ score,
-    __half *__restrict__ s16, float *__restrict__ s32, unsigned long long *trace, int T,
+    __half *__restrict__ s16, float *__restrict__ s32, __half *__restrict__ s16m,
+    __half *__restrict__ ssum, unsigned long long *trace, int T,
     uint32_t *__restrict__ bits, int wt, const float *__restrict__ r_in) {
   if (bits) dispatch_clear_part(T, bits, wt, blockIdx.y * E + blockIdx.x, E * T);
   router_block(blockIdx.x, blockIdx.y, x, xadd, norm_w, router, bias, has_bias, logits, sig,
-               score, s16, s32, trace, r_in);
+               score, s16, s32, s16m, ssum, trace, r_in);
 }
 
 // ---------------------------------------------------------------------------
@@ -198,20 +199,15 @@ template __global__ void HY3X_ROUTER_GEMM(LARGE)(const float *, const float *, i
 template __global__ void HY3X_ROUTER_GEMM(XL)(const float *, const float *, int, float *);
 template __global__ void HY3X_ROUTER_GEMM(XXL)(const float *, const float *, int, float *);
 
-// Routing of one token per wave (T > 1 paths), a block holding 1 or 4 waves: sigmoid and
-// score of the 192 logits (expert lane + 64 m in slot m), the top-K in
-// registers (topk_wave_fast, or topk_wave_regs on a tie or NaN), then the
-// token's bit in each of its experts' dispatch bitmaps.
-__global__ __launch_bounds__(256) void k_topk(const float *__restrict__ logits,
-                                              const float *__restrict__ bias, int has_bias, int K,
-                                              float scale, int T, int32_t *__restrict__ ids,
-                                              float *__restrict__ wpre, float *__restrict__ wout,
-                                              uint32_t *__restrict__ bits, int wt,
-                                              uint8_t *__restrict__ ranks) {
+// Routing of token t in one wave: sigmoid and score of the 192 logits (expert
+// lane + 64 m in slot m), the top-K in registers (topk_wave_fast, or
+// topk_wave_regs on a tie or NaN). Returns lane k's expert (k < K).
+__device__ __forceinline__ int route_token(const float *__restrict__ logits,
+                                           const float *__restrict__ bias, int has_bias, int K,
+                                           float scale, int t, int32_t *__restrict__ ids,
+                                           float *__restrict__ wpre, float *__restrict__ wout) {
 #pragma clang fp contract(off)
   const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (t >= T) return;  // whole waves
   float sg[3], sc[3];
 #pragma unroll
   for (int m = 0; m < 3; m++) {
@@ -234,6 +230,21 @@ __global__ __launch_bounds__(256) void k_topk(const float *__restrict__ logits,
     topk_wave_regs(sc, sg, K, scale, ids_t, wpre + (size_t)t * K, wout + (size_t)t * K);
     my_e = lane < K ? ids_t[lane] : 0;  // this lane's own store: program order
   }
+  return my_e;
+}
+
+// Top-K of one token per wave (more than ROUTE_SMALL_T tokens), a block holding
+// 1 or 4 waves, then the token's bit in each of its experts' dispatch bitmaps.
+__global__ __launch_bounds__(256) void k_topk(const float *__restrict__ logits,
+                                              const float *__restrict__ bias, int has_bias, int K,
+                                              float scale, int T, int32_t *__restrict__ ids,
+                                              float *__restrict__ wpre, float *__restrict__ wout,
+                                              uint32_t *__restrict__ bits, int wt,
+                                              uint8_t *__restrict__ ranks) {
+  const int lane = threadIdx.x & 63;
+  const int t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  if (t >= T) return;  // whole waves
+  const int my_e = route_token(logits, bias, has_bias, K, scale, t, ids, wpre, wout);
   if (bits && lane < K) {
     atomicOr(&bits[(size_t)my_e * wt + (t >> 5)], 1u << (t & 31));
     ranks[(size_t)my_e * wt * 32 + t] = (uint8_t)lane;  // lane k holds place k
@@ -246,6 +257,7 @@ __global__ __launch_bounds__(256) void k_topk(const float *__restrict__ logits,
 // expert's slots are listed in token order, so the lists (and the tiles, and
 // every result computed from them) do not depend on scheduling.
 // tiles[i] = {expert, first list index, count <= NT, 0}.
+// Exclusive scan over a block of 256 threads or more (tmp: one entry per wave).
 __device__ __forceinline__ int block_exclusive_scan256(int v, int *tmp) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   int incl = v;
@@ -260,6 +272,60 @@ __device__ __forceinline__ int block_exclusive_scan256(int v, int *tmp) {
   for (int w = 0; w < wave; w++) base += tmp[w];
   __syncthreads();
   return base + incl - v;
+}
+
+// Top-K and dispatch lists of up to ROUTE_SMALL_T tokens in one block of 512
+// threads: a wave routes a token (launch latency bounds this step, not work; as
+// k_topk and k_dispatch_list it was two launches, with a third that staged s),
+// marks the token in its experts' bitmaps in LDS, and thread e < 192 lists
+// expert e's slots in token order: the lists and tiles of k_dispatch_list.
+__global__ __launch_bounds__(64 * ROUTE_SMALL_T) void k_route_small(
+    const float *__restrict__ logits, const float *__restrict__ bias, int has_bias, int K,
+    float scale, int T, int NT, int32_t *__restrict__ ids, float *__restrict__ wpre,
+    float *__restrict__ wout, int32_t *__restrict__ list, int4 *__restrict__ tiles,
+    int32_t *__restrict__ n_tiles, int max_tiles, int32_t *__restrict__ counts_out,
+    unsigned long long *__restrict__ stats) {
+  static_assert(ROUTE_SMALL_T <= 8 && 64 * ROUTE_SMALL_T >= 256, "masks and packed scan");
+  __shared__ uint32_t mask[E];                    // expert e's tokens
+  __shared__ uint8_t place[E * ROUTE_SMALL_T];    // token t's place of expert e
+  __shared__ int tmp[ROUTE_SMALL_T];
+  const int tid = threadIdx.x, lane = tid & 63, t = tid >> 6;
+  if (tid < E) mask[tid] = 0u;
+  __syncthreads();
+  if (t < T) {
+    const int my_e = route_token(logits, bias, has_bias, K, scale, t, ids, wpre, wout);
+    if (lane < K) {
+      atomicOr(&mask[my_e], 1u << t);
+      place[my_e * ROUTE_SMALL_T + t] = (uint8_t)lane;
+    }
+  }
+  __syncthreads();
+  // slots, tiles and touched experts before expert tid (thread E: the shared
+  // expert), scanned together: all three counts stay below 1024
+  uint32_t m = tid < E ? mask[tid] : 0u;
+  const int c = tid == E ? T : __popc(m), nt = (c + NT - 1) / NT;
+  const int before = block_exclusive_scan256(c | nt << 10 | (c > 0) << 20, tmp);
+  const int off = before & 1023, toff = (before >> 10) & 1023;
+  if (tid <= E) {
+    if (counts_out) counts_out[tid] = c;
+    for (int j = 0; j < nt; j++)
+      if (toff + j < max_tiles)
+        tiles[toff + j] = make_int4(tid, off + j * NT, min(NT, c - j * NT), 0);
+  }
+  if (tid < E) {
+    for (int r = off; m; r++) {
+      const int tt = __ffs(m) - 1;
+      m &= m - 1u;
+      list[r] = tt * K + place[tid * ROUTE_SMALL_T + tt];
+    }
+  } else if (tid == E) {
+    for (int tt = 0; tt < T; tt++) list[off + tt] = T * K + tt;
+    *n_tiles = min(toff + nt, max_tiles);
+    if (stats) {  // forwards, experts touched (shared included)
+      stats[0] += 1ull;
+      stats[1] += (unsigned long long)((before >> 20) + 1);
+    }
+  }
 }
 
 // Dispatch lists from the bitmaps k_topk marked, one block per expert (E + 1

@@ -34,7 +34,7 @@ __global__ __launch_bounds__(256) void k_route_decode(
   const int tid = threadIdx.x;
   if (blockIdx.x < E) {
     router_block(blockIdx.x, 0, x, xadd, norm_w, router, bias, has_bias, logits, sig, score, s16,
-                 s32, trace, r_in);
+                 s32, nullptr, nullptr, trace, r_in);
     return;
   }
   // shared expert: s = rmsnorm(x) * norm_w, pair-staged fp16 in LDS. The

@@ -6,6 +6,7 @@
 #pragma once
 #include "hy3x_kernels.h"
 #include "hy3x_route.h"
+#include "hy3x_q4k.h"
 
 namespace hy3x {
 
@@ -49,13 +50,16 @@ __device__ __forceinline__ float chain_lanes(const float *rs, const float *xs, i
 // Small T: one block per (expert, token). The block stages x, norm_w and the
 // router row in LDS transposed by chain (buf[v][i] = a[8i+v]), reduces the
 // sum of squares in the fixed block order, then wave 0 runs the eight logit
-// chains (chain_lanes). Block (0, t) also stages s for the expert kernels.
+// chains (chain_lanes). Block (0, t) also stages s for the expert kernels: as
+// the MFMA tiles' operand and its sub-block sums (s16m, ssum) where those are
+// given, else pair-staged and in fp32 (s16, s32).
 __device__ __forceinline__ void router_block(
     int e, int t, const float *__restrict__ x, const float *__restrict__ xadd,
     const float *__restrict__ norm_w, const float *__restrict__ router,
     const float *__restrict__ bias, int has_bias, float *__restrict__ logits,
     float *__restrict__ sig, float *__restrict__ score, __half *__restrict__ s16,
-    float *__restrict__ s32, unsigned long long *trace, const float *__restrict__ r_in) {
+    float *__restrict__ s32, __half *__restrict__ s16m, __half *__restrict__ ssum,
+    unsigned long long *trace, const float *__restrict__ r_in) {
 #pragma clang fp contract(off)
   __shared__ __attribute__((aligned(16))) float xsf[8 * RS], rsf[8 * RS];
   const int tid = threadIdx.x;
@@ -106,6 +110,27 @@ __device__ __forceinline__ void router_block(
       score[(size_t)t * E + e] = has_bias ? sg + bias[e] : sg;
     }
     trace_point(trace, 3);
+  } else if (e == 0 && s16m) {
+    // waves 1 and 2, a sub-block of 32 per thread: fp16 in the MFMA run order
+    // (perm8) and the sub-block's sum, as k_rmsnorm and row_subsums form them
+    const int j = tid - 64;
+    if (j < D / 32) {
+      uint32_t w[16];
+#pragma unroll
+      for (int r = 0; r < 4; r++) {  // element 32 j + 8 r + q is xsf[q RS + 4 j + r]
+        const float *v = xsf + 4 * j + r;
+        const int q[8] = {0, 2, 1, 3, 4, 6, 5, 7};
+#pragma unroll
+        for (int u = 0; u < 4; u++)
+          w[4 * r + u] = __builtin_bit_cast(
+              uint32_t, (h2_t){(_Float16)v[q[2 * u] * RS], (_Float16)v[q[2 * u + 1] * RS]});
+      }
+      uint4 *dst = reinterpret_cast<uint4 *>(s16m + (size_t)t * D + 32 * j);
+#pragma unroll
+      for (int r = 0; r < 4; r++)
+        dst[r] = make_uint4(w[4 * r], w[4 * r + 1], w[4 * r + 2], w[4 * r + 3]);
+      store_subsum(ssum + (size_t)t * (D / 32) * 4, j, subsum16(w));
+    }
   } else if (e == 0 && tid >= 64) {
     // stage s for the expert kernels (fp16 pair-staged and fp32) from the
     // waves that run no chain

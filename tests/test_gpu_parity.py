@@ -182,6 +182,37 @@ def test_default_path_thresholds(torch, layer, cpu, T):
     assert O.rel_l2(y[rows] - x[rows], yo - x[rows]) <= TOL
 
 
+@pytest.mark.parametrize("kind", ["uniform", "hot", "ties"])
+@pytest.mark.parametrize("T,K,path", [(2, 1, 0), (2, 8, 0), (7, 3, 0), (8, 8, 0), (8, 8, 1)])
+def test_small_batch_lists(torch, layer, cpu, T, K, path, kind):
+    """Up to 8 tokens one block routes and makes the dispatch lists: evenly
+    spread tokens, every token on the same eight experts (GEMV tiles of 4
+    tokens: two tiles per expert), and those eight tied (a bias that absorbs
+    the sigmoids, so the selection with swaps decides). Routing bit-exact,
+    outputs against the oracle, the touched experts counted."""
+    nw, rt, b = C.layer_small_tensors(C.WEIGHT_SEED)
+    b = b.copy()
+    if kind != "uniform":
+        b[[5, 17, 60, 61, 99, 130, 171, 191]] = 50.0 if kind == "hot" else 1e8
+    saved, cpu.bias = cpu.bias, b
+    layer.set_router(nw, rt, b)
+    layer.set_path(path)
+    try:
+        x = C.inputs(0xCA, T)
+        layer.stats()
+        y, ids, wpre, w = run(torch, layer, x, K)
+        assert layer.stats() == (1, C.unique_experts(ids))
+        yo, ro = cpu.forward(x, K=K)
+    finally:
+        layer.set_path(0)
+        layer.set_router(nw, rt, C.layer_small_tensors(C.WEIGHT_SEED)[2])
+        cpu.bias = saved
+    assert np.array_equal(ids, ro["ids"])
+    assert np.array_equal(wpre.view(np.uint32), ro["wpre"].view(np.uint32))
+    assert np.array_equal(w.view(np.uint32), ro["w"].view(np.uint32))
+    assert O.rel_l2(y - x, yo - x) <= TOL
+
+
 def test_routing_without_bias(torch, layer, cpu):
     set_bias(layer, cpu, "none")
     x = C.inputs(0xC1, 12)
