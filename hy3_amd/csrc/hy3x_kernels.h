@@ -71,19 +71,22 @@ __global__ void k_topk(const float *logits, const float *bias, int has_bias, int
                        uint8_t *ranks);
 __global__ void k_dispatch_list(const uint8_t *ranks, int T, int K, int NT, const uint32_t *bits,
                                 int wt, int32_t *list, int4 *tiles,
-                                int32_t *n_tiles, int max_tiles, int32_t *counts_out,
+                                int32_t *n_tiles, int max_tiles, int NT2, int4 *tiles2,
+                                int32_t *n_tiles2, int32_t *counts_out,
                                 unsigned long long *stats);
 // Up to this many tokens one block routes every token and makes the dispatch
 // lists (k_route_small), in one launch where top-K, staging and dispatch were
 // three: 2 / 3 / 4 / 8 tokens 73.4 / 99.5 / 108.0 / 155.9 -> 64.4 / 90.0 / 98.3 /
 // 145.9 us per forward. It ends where the router stops running one wave per
 // (expert, token) and one wave per token still fits one block; the T > 8 router
-// stages s in k_rmsnorm and its dispatch alone takes about 4 us.
+// stages s in k_rmsnorm and its dispatch alone takes about 4 us. tiles2: the
+// down GEMM's list, of at most NT2 tokens per tile (0: none).
 constexpr int ROUTE_SMALL_T = 8;
 __global__ void k_route_small(const float *logits, const float *bias, int has_bias, int K,
                               float scale, int T, int NT, int32_t *ids, float *wpre, float *wout,
                               int32_t *list, int4 *tiles, int32_t *n_tiles, int max_tiles,
-                              int32_t *counts_out, unsigned long long *stats);
+                              int NT2, int4 *tiles2, int32_t *n_tiles2, int32_t *counts_out,
+                              unsigned long long *stats);
 template <int NT>
 __global__ void k_gateup_gemv(const uint8_t *wq, const __half *s16, const int32_t *list,
                               const int4 *tiles, const int32_t *n_tiles, int T, int K,
@@ -125,10 +128,12 @@ extern template __global__ void k_down_gemv<4>(const uint8_t *, const __half *, 
 // Tiles of grid margin for the kernels that deal whole tiles round-robin to
 // the XCDs (xcd_tile_rr, hy3x_mfma_ops.h).
 constexpr int XCD_TILE_RR_MARGIN = 7;
-// The MFMA grouped GEMMs in two shapes (hy3x_mfma.hip, compiled once per
+// The MFMA grouped GEMMs in three shapes (hy3x_mfma.hip, compiled once per
 // shape). A work tile has ROWS_GU = 16 WAVES RGU gate/up rows (per matrix) or
 // twice as many down rows and up to TOKENS tokens; each wave takes 16 RGU
 // gate/up rows or 32 RGU down rows:
+//   tiny:   8 tokens, 4 waves -- three workgroups per CU (46 KB of LDS); gate/up
+//           of a few tokens;
 //   narrow: 32 tokens, 4 waves -- two workgroups per CU; the shape for few
 //           tokens per expert;
 //   wide:   64 tokens, 8 waves -- one workgroup per CU, half the per-token
@@ -148,6 +153,7 @@ constexpr int XCD_TILE_RR_MARGIN = 7;
       const uint8_t *, const uint8_t *, const __half *, const __half *, const int32_t *,    \
       const int4 *, const int32_t *, int, int, __half *, float *);                          \
   }
+HY3X_DECLARE_MFMA(mfma_tiny, 8, 4, 1)
 HY3X_DECLARE_MFMA(mfma_narrow, 32, 4, 1)
 HY3X_DECLARE_MFMA(mfma_wide, 64, 8, 1)
 #undef HY3X_DECLARE_MFMA
@@ -170,6 +176,12 @@ extern template __global__ void k_moe_big<false>(const uint8_t *, const uint8_t 
                                                  const int32_t *, const int4 *, const int32_t *,
                                                  int, int, __half *, float *);
 }  // namespace mfma_big
+// The down GEMM for few tokens per expert (hy3x_mfma_few.hip): work tiles of
+// 16 FEW_WAVES rows and up to FEW_TOKENS tokens.
+constexpr int FEW_TOKENS = 4, FEW_WAVES = 4;
+__global__ void k_down_few(const uint8_t *wq, const uint8_t *wsh, const __half *act,
+                           const __half *act_sum, const int32_t *list, const int4 *tiles,
+                           const int32_t *n_tiles, float *out);
 __global__ void k_hsums(const __half *h16m, __half *hsum);
 
 __global__ void k_synth_q4k(uint8_t *dst, int64_t nblocks, uint64_t seed, uint32_t layer,

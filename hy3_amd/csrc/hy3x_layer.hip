@@ -41,7 +41,8 @@ struct Scratch {
   __half *s16 = nullptr, *h16 = nullptr, *s16m = nullptr, *h16m = nullptr;
   __half *ssum = nullptr, *hsum = nullptr;  // sub-block sums (hi, lo) of s16m / h16m rows
   int32_t *ids = nullptr, *list = nullptr, *n_tiles = nullptr, *counts = nullptr;
-  int4 *tiles = nullptr;
+  int4 *tiles = nullptr, *tiles2 = nullptr;
+  int32_t *n_tiles2 = nullptr;  // the down GEMM's own tile list (k_down_few)
   uint32_t *bits = nullptr;  // dispatch: per-expert token bitmaps [E][wt]
   uint8_t *ranks = nullptr;  // dispatch: [E][32 wt] token t's place of expert e where t's bit is set
 };
@@ -78,6 +79,8 @@ struct hy3x_layer {
     Mode mode = Mode::GEMV;
     bool wide = false;  // MFMA mode: the wide tile shape (mfma_wide)
     bool big = false;   // MFMA mode: 128-token tiles (mfma_big)
+    bool tiny = false;  // MFMA mode: gate/up in 8-token tiles (mfma_tiny)
+    bool few = false;   // MFMA mode: down by k_down_few
     const float *r_in = nullptr;  // substituted RMSNorm scales, or null
     Scratch sc;         // the scratch this forward runs on
     const hy3x_layer **owner = nullptr;  // that scratch's last-forward owner slot
@@ -173,6 +176,19 @@ constexpr int kXLRouterT = kRouterClassT[3];
 // T=32: 442 vs 550 us for gate/up + down), so the GEMV tiles only run when selected
 // explicitly (hy3x_layer_set_path 1); T = 1 keeps the fused decode kernels.
 constexpr int kMfmaMinT = 2;
+// Up to 8 tokens, gate/up runs in the 8-token shape (mfma_tiny: three workgroups
+// per CU, 768 in all, against the narrow shape's 512) where the routed experts'
+// row tiles, if no two tokens share one, overfill one round of the narrow shape
+// but about fill one of these: a second round for a few of them costs a whole
+// item's 16 columns. Gate/up us, narrow vs 8-token shape, K = 8: 2 tokens 29.7
+// vs 30.2, 3: 49.5 vs 45.0, 4: 53.7 vs 48.8, 5: 58.0 vs 62.6, 6: 66.6 vs 70.5, 8:
+// 80.1 vs 75-83.
+constexpr int kTinyMinRowTiles = 512, kTinyMaxRowTiles = 800;
+// Up to this many tokens the down GEMM keeps whole rows in registers
+// (k_down_few); above it the MFMA tiles' reuse of the dequantised weights wins.
+// Down launch us, narrow tiles vs whole rows: 2 tokens 19.4 vs 15.2, 8: 43.7 vs
+// 37.2, 16: 71.1 vs 57.7, 32: 91.0 vs 81.0, 48: 106.8 vs 101.7, 64: 116.1 vs 121.5.
+constexpr int kDownFewMaxT = 48;
 // From this many tokens the MFMA GEMMs use the wide tile shape (64 tokens, 8 waves).
 // Measured on MI355X (ms per layer, narrow vs wide): 32 tokens 0.32 vs 0.37,
 // 128: 0.43 vs 0.48, 256: 0.503 vs 0.517, 320: 0.556 vs 0.554, 384: 0.598 vs
@@ -196,7 +212,7 @@ static constexpr int max_tiles_for(int T, int K, int NT) {
 // max_tokens tokens (slots = tokens x (K_MAX routed + 1 shared)).
 enum ScratchPiece {
   SP_LOGITS, SP_SIG, SP_SCORE, SP_WPRE, SP_W, SP_IDS, SP_S16, SP_S32, SP_S16M, SP_H16M,
-  SP_SSUM, SP_HSUM, SP_H16, SP_OUT, SP_LIST, SP_TILES, SP_NTILES, SP_COUNTS, SP_BITS, SP_RANKS,
+  SP_SSUM, SP_HSUM, SP_H16, SP_OUT, SP_LIST, SP_TILES, SP_TILES2, SP_NTILES, SP_NTILES2, SP_COUNTS, SP_BITS, SP_RANKS,
   SP_COUNT
 };
 constexpr int bitmap_words(int max_tokens) { return ((max_tokens + 31) / 32 + 3) & ~3; }
@@ -214,7 +230,10 @@ constexpr size_t piece_bytes(int max_tokens, int piece) {
     case SP_OUT: return slots * D * sizeof(float);
     case SP_LIST: return slots * sizeof(int32_t);
     case SP_TILES: return (size_t)max_tiles_for(max_tokens, KMAX, 1) * sizeof(int4);
-    case SP_NTILES: return sizeof(int32_t);
+    case SP_TILES2:
+      return (size_t)max_tiles_for((int)std::min(T, (size_t)kDownFewMaxT), KMAX, FEW_TOKENS) *
+             sizeof(int4);
+    case SP_NTILES: case SP_NTILES2: return sizeof(int32_t);
     case SP_COUNTS: return (E + 1) * sizeof(int32_t);
     case SP_BITS: return (size_t)E * bitmap_words(max_tokens) * sizeof(uint32_t);
     case SP_RANKS: return (size_t)E * bitmap_words(max_tokens) * 32;
@@ -255,6 +274,8 @@ static Scratch scratch_layout(int max_tokens, uint8_t *base) {
   S.list = (int32_t *)p[SP_LIST];
   S.tiles = (int4 *)p[SP_TILES];
   S.n_tiles = (int32_t *)p[SP_NTILES];
+  S.tiles2 = (int4 *)p[SP_TILES2];
+  S.n_tiles2 = (int32_t *)p[SP_NTILES2];
   S.counts = (int32_t *)p[SP_COUNTS];
   S.bits = (uint32_t *)p[SP_BITS];
   S.ranks = (uint8_t *)p[SP_RANKS];
@@ -536,7 +557,8 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
       if (T <= ROUTE_SMALL_T) {
         k_route_small<<<1, 64 * ROUTE_SMALL_T, 0, st>>>(
             S.logits, L->bias, L->has_bias, K, c.scale, T, c.nt, S.ids, S.wpre, S.w, S.list,
-            S.tiles, S.n_tiles, mt, S.counts, L->stats);
+            S.tiles, S.n_tiles, mt, c.few ? FEW_TOKENS : 0, S.tiles2, S.n_tiles2, S.counts,
+            L->stats);
       } else {
         // one wave per token; up to 256 tokens one wave per block, so that
         // few tokens still spread over many CUs
@@ -549,8 +571,9 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
     case HY3X_STAGE_DISPATCH:
       if (c.mode != Mode::DECODE && T > ROUTE_SMALL_T) {
         k_dispatch_list<<<E + 1, 256, 0, st>>>(S.ranks, T, K, c.nt, S.bits, S.wt,
-                                               S.list, S.tiles, S.n_tiles, mt, S.counts,
-                                               L->stats);
+                                               S.list, S.tiles, S.n_tiles, mt,
+                                               c.few ? FEW_TOKENS : 0, S.tiles2, S.n_tiles2,
+                                               S.counts, L->stats);
       }
       break;
     case HY3X_STAGE_GATEUP:
@@ -558,6 +581,11 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
         k_gateup_decode<<<K * DEC_GU_BLOCKS, 64 * DEC_GU_WAVES, 0, st>>>(L->wq, S.s16, S.sig, S.score, K,
                                                           c.scale, S.ids, S.wpre, S.w,
                                                           L->stats, S.h16, L->trace[1]);
+      else if (c.mode == Mode::MFMA && c.tiny)
+        mfma_tiny::k_moe_mfma<true>
+            <<<mt * (F / mfma_tiny::ROWS_GU), 64 * mfma_tiny::WAVES, 0, st>>>(
+                L->wq, L->shared_q8 ? L->wsh : nullptr, S.s16m, S.ssum, S.list, S.tiles,
+                S.n_tiles, T, K, S.h16m, nullptr);
       else if (c.mode == Mode::MFMA && c.big)
         mfma_big::k_moe_big<true><<<(mt + XCD_TILE_RR_MARGIN) * (F / (16 * BIG_WAVES)), 64 * BIG_WAVES, 0, st>>>(
             L->wq, L->shared_q8 ? L->wsh : nullptr, S.s16m, S.ssum, S.list, S.tiles, S.n_tiles, T, K, S.h16m, nullptr);
@@ -583,7 +611,10 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
       else if (c.mode == Mode::MFMA) {
         k_hsums<<<T * (K + 1), 64, 0, st>>>(S.h16m, S.hsum);
         const uint8_t *wsh = L->shared_q8 ? L->wsh : nullptr;
-        if (c.big)
+        if (c.few)
+          k_down_few<<<max_tiles_for(T, K, FEW_TOKENS) * (D / (16 * FEW_WAVES)), 64 * FEW_WAVES,
+                       0, st>>>(L->wq, wsh, S.h16m, S.hsum, S.list, S.tiles2, S.n_tiles2, S.out);
+        else if (c.big)
           mfma_big::k_moe_big<false><<<mt * (D / (32 * BIG_WAVES)), 64 * BIG_WAVES, 0, st>>>(
               L->wq, wsh, S.h16m, S.hsum, S.list, S.tiles, S.n_tiles, T, K, nullptr, S.out);
         else if (c.wide)
@@ -674,6 +705,11 @@ static int forward_impl(hy3x_layer *L, const Scratch *sc, const hy3x_layer **own
           (L->path == 5 || ((L->path == 0 || L->path == 2) && T >= kMfmaBigMinT));
   c.wide = c.mode == Mode::MFMA && !c.big &&
            (L->path == 4 || (L->path != 3 && T >= kMfmaWideMinT));
+  const bool by_t = c.mode == Mode::MFMA && (L->path == 0 || L->path == 2);
+  const int row_tiles = (T * K + 1) * (F / mfma_tiny::ROWS_GU);
+  c.tiny = by_t && T <= mfma_tiny::TOKENS && row_tiles > kTinyMinRowTiles &&
+           row_tiles <= kTinyMaxRowTiles;
+  c.few = by_t && T <= kDownFewMaxT;
   // tokens per work tile
   c.nt = c.mode != Mode::MFMA ? 4
          : c.big              ? BIG_TOKENS

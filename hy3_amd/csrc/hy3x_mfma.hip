@@ -42,16 +42,19 @@
 
 namespace hy3x {
 
-// This file is compiled twice: as the narrow shape (namespace mfma_narrow)
-// and, with HY3X_MFMA_WIDE defined (hy3x_mfma_wide.hip), as the wide one.
-#ifdef HY3X_MFMA_WIDE
+// This file is compiled three times: as the narrow shape (namespace
+// mfma_narrow), with HY3X_MFMA_WIDE defined (hy3x_mfma_wide.hip) as the wide
+// one, and with HY3X_MFMA_TINY (hy3x_mfma_tiny.hip) as the 8-token one.
+#if defined(HY3X_MFMA_WIDE)
 namespace mfma_wide {
+#elif defined(HY3X_MFMA_TINY)
+namespace mfma_tiny {
 #else
 namespace mfma_narrow {
 #endif
 
 constexpr int MT_TOK = TOKENS;             // tokens per tile (dispatch NT for this path)
-static_assert(MT_TOK == 32 || MT_TOK == 64, "tile tokens");
+static_assert(MT_TOK == 8 || MT_TOK == 32 || MT_TOK == 64, "tile tokens");
 constexpr int MT_WAVES = WAVES;            // waves per workgroup
 constexpr int MT_THREADS = 64 * MT_WAVES;
 constexpr int MT_RGU = RGU;                // 16-row gate/up groups per wave (down: twice)
@@ -78,6 +81,10 @@ __shared__ __attribute__((aligned(16))) u4_t a_ring[A_STAGES][A_CHUNKS];
 __shared__ __attribute__((aligned(16))) u4_t bt_st[2][MT_TOK][32];
 __shared__ __attribute__((aligned(16))) u4_t bm_st[2][MT_TOK][4];
 __shared__ int32_t t_slot[MT_TOK], t_arow[MT_TOK];
+// The LDS row of MFMA row r (the 8-token shape's MFMA rows 8 .. 15, whose
+// results are never stored, read its rows again).
+__device__ __forceinline__ int tok_row(int r) { return r & (MT_TOK - 1); }
+__device__ __forceinline__ int swz(int lr) { return lr & (MT_TOK < 16 ? MT_TOK - 1 : 15); }
 
 template <bool GATEUP>
 struct MfmaCfg {
@@ -261,9 +268,9 @@ __device__ __forceinline__ void mfma_step(TileState<GATEUP, NTT> &st, int kb) {
     for (int i = 0; i < 8; i++) {
       // MFMA i = 4 piece + 2 h + u: k0 = 128 piece + 32 h + 8 u + 64 (g>>1) + 16 (g&1)
       const int c = 16 * (i >> 2) + 4 * ((i >> 1) & 1) + (i & 1) + gch;
-      x[t][i] = __builtin_bit_cast(h8_t, bt_st[buf][16 * t + lr][c ^ lr]);
+      x[t][i] = __builtin_bit_cast(h8_t, bt_st[buf][tok_row(16 * t + lr)][c ^ swz(lr)]);
     }
-    sv[t] = __builtin_bit_cast(h8_t, bm_st[buf][16 * t + lr][g ^ ((lr >> 2) & 3)]);
+    sv[t] = __builtin_bit_cast(h8_t, bm_st[buf][tok_row(16 * t + lr)][g ^ ((swz(lr) >> 2) & 3)]);
   }
 
   // the previous column's d * Dblk, in the same order on acc as if it had
@@ -424,7 +431,7 @@ __device__ __forceinline__ void mfma_tile(const uint8_t *__restrict__ wq,
 // permute, minus 1152) and each block's MFMA result is scaled by its d in
 // fp32: acc += d_b * (x_b . q_b) -- sum d*q*x as mul_mat_f32 case 8
 // (hy3.c:1098-1120).
-constexpr int B8_DMA = MT_TOK * 16 / 64 / MT_WAVES;  // activation copies per wave
+constexpr int B8_DMA = MT_TOK < 16 ? 1 : MT_TOK * 16 / 64 / MT_WAVES;  // activation copies per wave
 
 template <bool GATEUP, int NTT>
 struct TileStateQ8 {
@@ -486,7 +493,7 @@ __device__ __forceinline__ void mfma_step_q8(TileStateQ8<GATEUP, NTT> &st, int k
   for (int t = 0; t < NTT; t++)
 #pragma unroll
     for (int b = 0; b < 4; b++)
-      x[t][b] = __builtin_bit_cast(h8_t, bt[16 * (16 * t + lr) + ((4 * b + g) ^ lr)]);
+      x[t][b] = __builtin_bit_cast(h8_t, bt[16 * tok_row(16 * t + lr) + ((4 * b + g) ^ swz(lr))]);
   const f4_t zero4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int b = 0; b < 4; b++) {
@@ -531,7 +538,7 @@ __device__ __forceinline__ void mfma_tile_q8(const uint8_t *__restrict__ wsh,
   st.bbase = reinterpret_cast<const uint8_t *>(act);
 #pragma unroll
   for (int j = 0; j < B8_DMA; j++) {
-    const int q = 64 * (B8_DMA * wave + j) + lane, r = q >> 4;
+    const int q = 64 * (B8_DMA * wave + j) + lane, r = tok_row(q >> 4);
     const int ar = t_arow[r] >= 0 ? t_arow[r] : arow0;
     st.boff[j] = (uint32_t)(2 * (ar * KD + 8 * ((q & 15) ^ (r & 15))));
   }
@@ -596,8 +603,8 @@ __global__ __launch_bounds__(MT_THREADS) void k_moe_mfma(
         return;
       }
     }
-    if (n > 16)
-      mfma_tile_q8<GATEUP, 2>(wsh, act, n, rt, h16m, out);
+    if (MT_TOK > 16 && n > 16)
+      mfma_tile_q8<GATEUP, (MT_TOK > 16 ? 2 : 1)>(wsh, act, n, rt, h16m, out);
     else
       mfma_tile_q8<GATEUP, 1>(wsh, act, n, rt, h16m, out);
     return;
@@ -612,8 +619,8 @@ __global__ __launch_bounds__(MT_THREADS) void k_moe_mfma(
       return;
     }
   }
-  if (n > 16)
-    mfma_tile<GATEUP, 2>(wq, act, act_sum, e, n, rt, h16m, out);
+  if (MT_TOK > 16 && n > 16)
+    mfma_tile<GATEUP, (MT_TOK > 16 ? 2 : 1)>(wq, act, act_sum, e, n, rt, h16m, out);
   else
     mfma_tile<GATEUP, 1>(wq, act, act_sum, e, n, rt, h16m, out);
 }
@@ -625,9 +632,9 @@ template __global__ void k_moe_mfma<false>(const uint8_t *, const uint8_t *, con
                                            const __half *, const int32_t *, const int4 *,
                                            const int32_t *, int, int, __half *, float *);
 
-}  // namespace mfma_narrow / mfma_wide
+}  // namespace mfma_narrow / mfma_wide / mfma_tiny
 
-#ifndef HY3X_MFMA_WIDE
+#if !defined(HY3X_MFMA_WIDE) && !defined(HY3X_MFMA_TINY)
 
 // The 48 sub-block sums of every h row (down-GEMM mins operand); one wave per slot.
 __global__ __launch_bounds__(64) void k_hsums(const __half *__restrict__ h16m,
@@ -636,6 +643,6 @@ __global__ __launch_bounds__(64) void k_hsums(const __half *__restrict__ h16m,
   row_subsums(h16m + (size_t)slot * F, F / 32, hsum + (size_t)slot * (F / 32) * 4);
 }
 
-#endif  // !HY3X_MFMA_WIDE
+#endif
 
 }  // namespace hy3x

@@ -283,7 +283,8 @@ __global__ __launch_bounds__(64 * ROUTE_SMALL_T) void k_route_small(
     const float *__restrict__ logits, const float *__restrict__ bias, int has_bias, int K,
     float scale, int T, int NT, int32_t *__restrict__ ids, float *__restrict__ wpre,
     float *__restrict__ wout, int32_t *__restrict__ list, int4 *__restrict__ tiles,
-    int32_t *__restrict__ n_tiles, int max_tiles, int32_t *__restrict__ counts_out,
+    int32_t *__restrict__ n_tiles, int max_tiles, int NT2, int4 *__restrict__ tiles2,
+    int32_t *__restrict__ n_tiles2, int32_t *__restrict__ counts_out,
     unsigned long long *__restrict__ stats) {
   static_assert(ROUTE_SMALL_T <= 8 && 64 * ROUTE_SMALL_T >= 256, "masks and packed scan");
   __shared__ uint32_t mask[E];                    // expert e's tokens
@@ -300,17 +301,20 @@ __global__ __launch_bounds__(64 * ROUTE_SMALL_T) void k_route_small(
     }
   }
   __syncthreads();
-  // slots, tiles and touched experts before expert tid (thread E: the shared
-  // expert), scanned together: all three counts stay below 1024
+  // slots, tiles of either list and touched experts before expert tid (thread E:
+  // the shared expert), scanned together: each count stays below 128
   uint32_t m = tid < E ? mask[tid] : 0u;
   const int c = tid == E ? T : __popc(m), nt = (c + NT - 1) / NT;
-  const int before = block_exclusive_scan256(c | nt << 10 | (c > 0) << 20, tmp);
-  const int off = before & 1023, toff = (before >> 10) & 1023;
+  const int nt2 = NT2 ? (c + NT2 - 1) / NT2 : 0;
+  const int before = block_exclusive_scan256(c | nt << 7 | nt2 << 14 | (c > 0) << 21, tmp);
+  const int off = before & 127, toff = (before >> 7) & 127, toff2 = (before >> 14) & 127;
   if (tid <= E) {
     if (counts_out) counts_out[tid] = c;
     for (int j = 0; j < nt; j++)
       if (toff + j < max_tiles)
         tiles[toff + j] = make_int4(tid, off + j * NT, min(NT, c - j * NT), 0);
+    for (int j = 0; j < nt2; j++)
+      tiles2[toff2 + j] = make_int4(tid, off + j * NT2, min(NT2, c - j * NT2), 0);
   }
   if (tid < E) {
     for (int r = off; m; r++) {
@@ -321,9 +325,10 @@ __global__ __launch_bounds__(64 * ROUTE_SMALL_T) void k_route_small(
   } else if (tid == E) {
     for (int tt = 0; tt < T; tt++) list[off + tt] = T * K + tt;
     *n_tiles = min(toff + nt, max_tiles);
+    if (NT2) *n_tiles2 = toff2 + nt2;
     if (stats) {  // forwards, experts touched (shared included)
       stats[0] += 1ull;
-      stats[1] += (unsigned long long)((before >> 20) + 1);
+      stats[1] += (unsigned long long)((before >> 21) + 1);
     }
   }
 }
@@ -331,11 +336,14 @@ __global__ __launch_bounds__(64 * ROUTE_SMALL_T) void k_route_small(
 // Dispatch lists from the bitmaps k_topk marked, one block per expert (E + 1
 // blocks, the last is the shared expert): list offset and first tile from exclusive scans of all counts, the expert's
 // tiles, and its slots in token order from its bitmap (popcount prefix sums).
-// Block E also writes the tile count, the per-expert counts and the stats.
+// NT2 != 0: a second tile list over the same slots, of at most NT2 tokens per
+// tile (the two lists' offsets are then scanned packed: fewer than 32768 tiles).
+// Block E also writes the tile counts, the per-expert counts and the stats.
 __global__ __launch_bounds__(256) void k_dispatch_list(
     const uint8_t *__restrict__ ranks, int T, int K, int NT, const uint32_t *__restrict__ bits,
     int wt, int32_t *__restrict__ list,
-    int4 *__restrict__ tiles, int32_t *__restrict__ n_tiles, int max_tiles,
+    int4 *__restrict__ tiles, int32_t *__restrict__ n_tiles, int max_tiles, int NT2,
+    int4 *__restrict__ tiles2, int32_t *__restrict__ n_tiles2,
     int32_t *__restrict__ counts_out, unsigned long long *__restrict__ stats) {
   __shared__ int tmp[8], off_l, toff_l, ce_l;
   const int e = blockIdx.x, tid = threadIdx.x;
@@ -353,17 +361,19 @@ __global__ __launch_bounds__(256) void k_dispatch_list(
     }
   }
   const int off = block_exclusive_scan256(c, tmp);
-  const int nt = (c + NT - 1) / NT;
-  const int toff = block_exclusive_scan256(nt, tmp);
+  const int nt = (c + NT - 1) / NT, nt2 = NT2 ? (c + NT2 - 1) / NT2 : 0;
+  const int toffs = block_exclusive_scan256(nt | nt2 << 16, tmp);
+  const int toff = NT2 ? toffs & 0xffff : toffs, toff2 = NT2 ? toffs >> 16 : 0;
   if (tid == e) {
     off_l = off;
-    toff_l = toff;
+    toff_l = toffs;
     ce_l = c;
   }
   if (e == E) {
     const int active = block_exclusive_scan256(c > 0 ? 1 : 0, tmp);
     if (tid == 255) {
       *n_tiles = toff < max_tiles ? toff : max_tiles;
+      if (NT2) *n_tiles2 = toff2;
       if (stats) {  // forwards, experts touched (shared included)
         stats[0] += 1ull;
         stats[1] += (unsigned long long)active;
@@ -372,9 +382,13 @@ __global__ __launch_bounds__(256) void k_dispatch_list(
     if (counts_out && tid <= E) counts_out[tid] = c;
   }
   __syncthreads();
-  const int eoff = off_l, etoff = toff_l, ce = ce_l;
+  const int eoff = off_l, ce = ce_l;
+  const int etoff = NT2 ? toff_l & 0xffff : toff_l, etoff2 = NT2 ? toff_l >> 16 : 0;
   for (int j = tid; j * NT < ce; j += 256)
     if (etoff + j < max_tiles) tiles[etoff + j] = make_int4(e, eoff + j * NT, min(NT, ce - j * NT), 0);
+  if (NT2)
+    for (int j = tid; j * NT2 < ce; j += 256)
+      tiles2[etoff2 + j] = make_int4(e, eoff + j * NT2, min(NT2, ce - j * NT2), 0);
   if (e == E) {
     for (int t = tid; t < T; t += 256) list[eoff + t] = T * K + t;
     return;

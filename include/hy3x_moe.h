@@ -250,7 +250,8 @@ int hy3x_layer_set_rms_scale(hy3x_layer *layer, const float *r, int n);
 int hy3x_layer_set_path(hy3x_layer *layer, int path);
 
 /* Which expert path the last forward ran: 0 = the fused single-token decode
- * kernels, 1 = wavefront-GEMV tiles, 3 = MFMA with the narrow tile shape,
+ * kernels, 1 = wavefront-GEMV tiles, 3 = MFMA with the narrow tile shape (by
+ * itself, path 0, with variants of it for few tokens that give the same bits),
  * 4 = MFMA with the wide one, 5 = MFMA with 128-token tiles (diagnostics and benchmarks: the kernel whose
  * roofline a benchmark reports). */
 int hy3x_layer_last_path(const hy3x_layer *layer, int *path);

@@ -578,6 +578,33 @@ def test_big_tiles_equal_narrow_tiles(torch, layer, cpu, T):
     assert np.array_equal(y3.view(np.uint32), y5.view(np.uint32))
 
 
+@pytest.mark.parametrize("hot", [False, True])
+@pytest.mark.parametrize("T,K", [(2, 8), (3, 8), (4, 8), (5, 3), (8, 4), (9, 8), (33, 8), (48, 8),
+                                 (49, 8)])
+def test_few_token_kernels_equal_narrow_tiles(torch, layer, T, K, hot):
+    """The kernels that serve few tokens by default -- the 8-token gate/up
+    tiles, where the row tiles overfill one round of the narrow shape (3 and 4
+    tokens at K = 8, 8 at K = 4), and the down GEMM with whole rows in registers
+    (up to 48 tokens, tiles of 4) -- give the narrow tiles' bits, evenly spread
+    and with every token on the same experts (full tiles and remainders)."""
+    nw, rt, b = C.layer_small_tensors(C.WEIGHT_SEED)
+    if hot:
+        b = b.copy()
+        b[[5, 17, 60, 61, 99, 130, 171, 191]] = 50.0
+    layer.set_router(nw, rt, b)
+    x = C.inputs(0xCB, T)
+    try:
+        y0, ids0, _, _ = run(torch, layer, x, K)
+        assert layer.last_path() == 3
+        layer.set_path(3)
+        y3, ids3, _, _ = run(torch, layer, x, K)
+    finally:
+        layer.set_path(0)
+        layer.set_router(nw, rt, C.layer_small_tensors(C.WEIGHT_SEED)[2])
+    assert np.array_equal(ids0, ids3)
+    assert np.array_equal(y0.view(np.uint32), y3.view(np.uint32))
+
+
 @pytest.mark.parametrize("T", [16, 40, 64, 128, 129, 200, 257])
 def test_mfma_tile_shapes_on_crowded_experts(torch, layer, cpu, T):
     """A bias of +50 on eight experts sends every token to them, so each of
@@ -753,6 +780,20 @@ def test_q8_shared_big_tiles_equal_narrow_tiles(torch, q8_layer, T):
         q8_layer.set_path(0)
     assert np.array_equal(y3.view(np.uint32), y5.view(np.uint32))
     assert np.array_equal(y3.view(np.uint32), y0.view(np.uint32))
+
+
+@pytest.mark.parametrize("T", [2, 3, 8, 20, 48])
+def test_q8_shared_few_token_kernels_equal_narrow_tiles(torch, q8_layer, T):
+    """The few-token kernels on the Q8_0 shared expert's tiles (several of 4
+    tokens each): the narrow tiles' bits."""
+    x = C.inputs(0xCC, T)
+    y0, *_ = run(torch, q8_layer, x)
+    try:
+        q8_layer.set_path(3)
+        y3, *_ = run(torch, q8_layer, x)
+    finally:
+        q8_layer.set_path(0)
+    assert np.array_equal(y0.view(np.uint32), y3.view(np.uint32))
 
 
 def test_q8_shared_reference_tokens(torch, q8_layer):
