@@ -181,7 +181,7 @@ extern template __global__ void k_moe_big<false>(const uint8_t *, const uint8_t 
 constexpr int FEW_TOKENS = 4, FEW_WAVES = 4;
 __global__ void k_down_few(const uint8_t *wq, const uint8_t *wsh, const __half *act,
                            const __half *act_sum, const int32_t *list, const int4 *tiles,
-                           const int32_t *n_tiles, float *out);
+                           const int32_t *n_tiles, int T, float *out);
 __global__ void k_hsums(const __half *h16m, __half *hsum);
 
 __global__ void k_synth_q4k(uint8_t *dst, int64_t nblocks, uint64_t seed, uint32_t layer,

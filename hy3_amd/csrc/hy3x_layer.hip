@@ -613,7 +613,7 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
         const uint8_t *wsh = L->shared_q8 ? L->wsh : nullptr;
         if (c.few)
           k_down_few<<<max_tiles_for(T, K, FEW_TOKENS) * (D / (16 * FEW_WAVES)), 64 * FEW_WAVES,
-                       0, st>>>(L->wq, wsh, S.h16m, S.hsum, S.list, S.tiles2, S.n_tiles2, S.out);
+                       0, st>>>(L->wq, wsh, S.h16m, S.hsum, S.list, S.tiles2, S.n_tiles2, T, S.out);
         else if (c.big)
           mfma_big::k_moe_big<false><<<mt * (D / (32 * BIG_WAVES)), 64 * BIG_WAVES, 0, st>>>(
               L->wq, wsh, S.h16m, S.hsum, S.list, S.tiles, S.n_tiles, T, K, nullptr, S.out);

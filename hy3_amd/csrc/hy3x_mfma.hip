@@ -580,7 +580,7 @@ __global__ __launch_bounds__(MT_THREADS) void k_moe_mfma(
   // share its weights in L2; whole tiles dealt round-robin measured equal at
   // 32 tokens and 0.7 % slower at 512)
   if ((int)blockIdx.x >= nreal) return;
-  const int w = xcd_remap(blockIdx.x, nreal);
+  const int w = xcd_remap(blockIdx.x, nreal, (T + MT_TOK - 1) / MT_TOK * C::NRT);
   const int tile = w / C::NRT, rt = w % C::NRT;
   const int4 td = tiles[tile];
   const int e = td.x, o = td.y, n = td.z;

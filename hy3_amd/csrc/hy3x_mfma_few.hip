@@ -37,13 +37,13 @@ __global__ __launch_bounds__(FW_THREADS, 4) void k_down_few(
     const uint8_t *__restrict__ wq, const uint8_t *__restrict__ wsh,
     const __half *__restrict__ act, const __half *__restrict__ act_sum,
     const int32_t *__restrict__ list, const int4 *__restrict__ tiles,
-    const int32_t *__restrict__ n_tiles, float *__restrict__ out) {
+    const int32_t *__restrict__ n_tiles, int T, float *__restrict__ out) {
   constexpr int TROWS = 16 * FEW_WAVES, NRT = D / TROWS;
   __shared__ __attribute__((aligned(16))) u4_t x_l[FEW_TOKENS * FW_XROW];
   __shared__ __attribute__((aligned(16))) u4_t s_l[FEW_TOKENS * FW_SROW];
   const int nreal = *n_tiles * NRT;
   if ((int)blockIdx.x >= nreal) return;
-  const int w = xcd_remap(blockIdx.x, nreal);
+  const int w = xcd_remap(blockIdx.x, nreal, (T + FEW_TOKENS - 1) / FEW_TOKENS * NRT);
   const int4 td = tiles[w / NRT];
   const int e = td.x, n = td.z;
   const int tid = threadIdx.x, lr = tid & 15, g = (tid >> 4) & 3;

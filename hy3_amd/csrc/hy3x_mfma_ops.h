@@ -113,13 +113,21 @@ __device__ __forceinline__ h8_t mins_operand(uint32_t hx, uint32_t mw, uint32_t 
   return (h8_t){hi[0], hi[1], hi[0], hi[1], lo[0], lo[1], lo[0], lo[1]};
 }
 
-// Launch order -> work item, so that consecutive work items run on one XCD
-// (workgroups are dealt to the 8 XCDs round-robin): the row tiles of one
-// expert tile share its activations in that XCD's L2, and consecutive token
-// tiles of one expert share its weights.
-__device__ __forceinline__ int xcd_remap(int bid, int nblocks) {
+// Launch order -> work item (workgroups are dealt to the 8 XCDs round-robin).
+// The first `shared` items, the shared expert's, go round the XCDs at the start
+// of the launch: with Q8 weights they take twice as long as a routed expert's,
+// and at the end of one XCD's work they were the launch's tail (8 tokens, Q8:
+// gate/up 95.7 us and down 46.8, first and spread 83.4 and 40.4; 20: 146.8 and
+// 86.5, 139.7 and 69.4). The rest: consecutive items on one XCD,
+// so that the row tiles of one expert tile share its activations in that XCD's
+// L2, and consecutive token tiles of one expert share its weights.
+__device__ __forceinline__ int xcd_remap(int bid, int nblocks, int shared) {
+  const int s8 = shared & ~7;
+  if (bid < s8) return bid;
+  nblocks -= s8;
+  bid -= s8;
   const int q = nblocks >> 3, r = nblocks & 7, x = bid & 7, i = bid >> 3;
-  return x * q + (x < r ? x : r) + i;
+  return s8 + x * q + (x < r ? x : r) + i;
 }
 
 // Launch order -> work item with whole tiles dealt round-robin to the XCDs:

@@ -256,7 +256,8 @@ __global__ __launch_bounds__(256) void k_topk(const float *__restrict__ logits,
 // token t of the shared expert (index E), which every token uses. Each
 // expert's slots are listed in token order, so the lists (and the tiles, and
 // every result computed from them) do not depend on scheduling.
-// tiles[i] = {expert, first list index, count <= NT, 0}.
+// tiles[i] = {expert, first list index, count <= NT, 0}: the shared expert's
+// tiles first (see xcd_remap), then the routed experts'.
 // Exclusive scan over a block of 256 threads or more (tmp: one entry per wave).
 __device__ __forceinline__ int block_exclusive_scan256(int v, int *tmp) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -310,11 +311,13 @@ __global__ __launch_bounds__(64 * ROUTE_SMALL_T) void k_route_small(
   const int off = before & 127, toff = (before >> 7) & 127, toff2 = (before >> 14) & 127;
   if (tid <= E) {
     if (counts_out) counts_out[tid] = c;
+    const int i0 = tid == E ? 0 : toff + (T + NT - 1) / NT;
+    const int i2 = tid == E ? 0 : toff2 + (T + NT2 - 1) / max(NT2, 1);
     for (int j = 0; j < nt; j++)
-      if (toff + j < max_tiles)
-        tiles[toff + j] = make_int4(tid, off + j * NT, min(NT, c - j * NT), 0);
+      if (i0 + j < max_tiles)
+        tiles[i0 + j] = make_int4(tid, off + j * NT, min(NT, c - j * NT), 0);
     for (int j = 0; j < nt2; j++)
-      tiles2[toff2 + j] = make_int4(tid, off + j * NT2, min(NT2, c - j * NT2), 0);
+      tiles2[i2 + j] = make_int4(tid, off + j * NT2, min(NT2, c - j * NT2), 0);
   }
   if (tid < E) {
     for (int r = off; m; r++) {
@@ -372,7 +375,7 @@ __global__ __launch_bounds__(256) void k_dispatch_list(
   if (e == E) {
     const int active = block_exclusive_scan256(c > 0 ? 1 : 0, tmp);
     if (tid == 255) {
-      *n_tiles = toff < max_tiles ? toff : max_tiles;
+      *n_tiles = toff < max_tiles ? toff : max_tiles;  // thread 255: after all experts
       if (NT2) *n_tiles2 = toff2;
       if (stats) {  // forwards, experts touched (shared included)
         stats[0] += 1ull;
@@ -383,7 +386,8 @@ __global__ __launch_bounds__(256) void k_dispatch_list(
   }
   __syncthreads();
   const int eoff = off_l, ce = ce_l;
-  const int etoff = NT2 ? toff_l & 0xffff : toff_l, etoff2 = NT2 ? toff_l >> 16 : 0;
+  const int etoff = e == E ? 0 : (NT2 ? toff_l & 0xffff : toff_l) + (T + NT - 1) / NT;
+  const int etoff2 = e == E || !NT2 ? 0 : (toff_l >> 16) + (T + NT2 - 1) / NT2;
   for (int j = tid; j * NT < ce; j += 256)
     if (etoff + j < max_tiles) tiles[etoff + j] = make_int4(e, eoff + j * NT, min(NT, ce - j * NT), 0);
   if (NT2)
