@@ -14,58 +14,40 @@ __global__ void k_rmsnorm(const float *x, const float *xadd, const float *norm_w
                           float *s32,
                           __half *s16m, __half *ssum, int T, uint32_t *bits, int wt,
                           const float *r_in);
-// Router GEMM tile shapes by token count (k_router_gemm<MT, ME, 4, 8, KC,
-// R>): a thread holds MT x ME (token, expert) outputs of one chain, a block
-// 4 MT tokens x 8 ME experts; K is walked in chunks of KC floats with R
-// chunks in flight. Few blocks run at small T, so there each chunk's load
-// latency must hide behind the previous chunks' FMAs; at large T the tile
-// sets the LDS reads per FMA and the block count per CU. Measured on MI355X
-// (router stage, RMSNorm + GEMM + top-K; the shape replaced in brackets):
-//   TINY  T <= 64:   4 x 8,   KC 256, R 2 (T = 32: 21.4 us; 4 x 16: 25.1, 4 x 24: 31.0)
-//   MID   T <= 256:  8 x 16,  KC 256, R 2 (T = 96 / 160 / 256: 28.5 / 28.8 / 36.4 us;
-//                    KC 128: 29.5 / 29.6 / 34.3, 8 x 24: 33.7 / 33.9 / 34.5)
-//   LARGE T <= 1536: 16 x 24, KC 128, R 1 (T = 512: 42.8 us [16 x 16: 49.3],
-//                    T = 1024: 62.4 us [32 x 32: 93.7], T = 1536: 86.3 [103.0];
-//                    T = 2048: 113.7 against 108.6 for 32 x 32)
-//   XL    T <= 2560: 32 x 32, KC 64,  R 4 (T = 2560: 115.0 us; 32 x 48: 138.5)
-//   XXL   T > 2560:  32 x 48, KC 64,  R 4 (T = 3072: 140.9 us [32 x 32: 147.2],
-//                    T = 4096: 155.9 [165.7])
-#define HY3X_RCFG(NAME, MT, ME, KC, R)                                                         \
-  constexpr int ROUTER_MT_##NAME = MT, ROUTER_ME_##NAME = ME, ROUTER_KC_##NAME = KC,        \
-                ROUTER_R_##NAME = R;
-#ifndef HY3X_RCFG_TINY
-#define HY3X_RCFG_TINY 1, 1, 256, 2
-#endif
-#ifndef HY3X_RCFG_MID
-#define HY3X_RCFG_MID 2, 2, 256, 2
-#endif
-#ifndef HY3X_RCFG_LARGE
-#define HY3X_RCFG_LARGE 4, 3, 128, 1
-#endif
-#ifndef HY3X_RCFG_XL
-#define HY3X_RCFG_XL 8, 4, 64, 4
-#endif
-#ifndef HY3X_RCFG_XXL
-#define HY3X_RCFG_XXL 8, 6, 64, 4
-#endif
-#define HY3X_RCFG_(NAME, ...) HY3X_RCFG(NAME, __VA_ARGS__)
-HY3X_RCFG_(TINY, HY3X_RCFG_TINY)
-HY3X_RCFG_(MID, HY3X_RCFG_MID)
-HY3X_RCFG_(LARGE, HY3X_RCFG_LARGE)
-HY3X_RCFG_(XL, HY3X_RCFG_XL)
-HY3X_RCFG_(XXL, HY3X_RCFG_XXL)
-#undef HY3X_RCFG_
-#undef HY3X_RCFG
+// Router GEMM shapes by token count, X(up to T, MT, ME, TG, KC, R): a thread of
+// k_router_gemm<MT, ME, TG, 8, KC, R> holds MT x ME (token, expert) outputs of one
+// chain, a block of 64 TG threads MT TG tokens x 8 ME experts; K is walked in chunks
+// of KC floats with R chunks in flight. Every block walks all of K at a pace set by
+// LDS latency and its barriers, so up to 1344 tokens the shape is the smallest tile
+// whose blocks fit the 256 CUs once (the boundaries: 240 to 256 blocks); eight waves
+// hide more of the latency than four where the tile's fetch splits that finely.
+// Router stage (RMSNorm + GEMM + top-K) on MI355X, us, the shape taken before (4 x 8
+// up to 64 tokens, 8 x 16 to 256, 16 x 24 to 1536, 32 x 32 in four waves to 2560, as
+// below above) in brackets:
+//   4 x 8    T = 40: 20.4 [22.0]           8 x 8    T = 64: 22.9 [28.2], 75: 23.2 [28.5]
+//   8 x 16   T = 160: 26.8 [29.2]          16 x 16  T = 201: 33.2 [36.1], 320: 35.2 [42.0]
+//   16 x 24  T = 512: 43.7 (16 x 16: 53.3) 16 x 32  T = 600: 44.7 [60.2]
+//   32 x 32  T = 1000: 60.6 [66.9], 1344: 64.6 [86.9] (KC 64, R 4: 73.5 at 1000); with KC
+//            64, R 4: T = 2048: 96.9 [112.5] (KC 128: 99.1), 2560: 108.8 [121.0]
+//   32 x 48  T = 4096: 164 (64 x 32: 197, 64 x 48 in eight waves: 186)
+#define HY3X_ROUTER_SHAPES(X)                                                                  \
+  X(40, 1, 1, 4, 256, 2)                                                                       \
+  X(80, 1, 1, 8, 256, 2)                                                                       \
+  X(168, 2, 2, 4, 256, 2)                                                                      \
+  X(336, 2, 2, 8, 128, 2)                                                                      \
+  X(512, 4, 3, 4, 128, 1)                                                                      \
+  X(672, 2, 4, 8, 128, 2)                                                                      \
+  X(1344, 4, 4, 8, 128, 2)                                                                     \
+  X(2560, 4, 4, 8, 64, 4)                                                                      \
+  X(INT32_MAX, 8, 6, 4, 64, 4)
 template <int MT, int ME, int TG, int EG, int KC, int R>
-__global__ __launch_bounds__(256) void k_router_gemm(const float *s32, const float *router, int T,
-                                                     float *logits);
-#define HY3X_ROUTER_GEMM(NAME)                                                                 \
-  k_router_gemm<ROUTER_MT_##NAME, ROUTER_ME_##NAME, 4, 8, ROUTER_KC_##NAME, ROUTER_R_##NAME>
-extern template __global__ void HY3X_ROUTER_GEMM(TINY)(const float *, const float *, int, float *);
-extern template __global__ void HY3X_ROUTER_GEMM(MID)(const float *, const float *, int, float *);
-extern template __global__ void HY3X_ROUTER_GEMM(LARGE)(const float *, const float *, int, float *);
-extern template __global__ void HY3X_ROUTER_GEMM(XL)(const float *, const float *, int, float *);
-extern template __global__ void HY3X_ROUTER_GEMM(XXL)(const float *, const float *, int, float *);
+__global__ __launch_bounds__(8 * TG * EG) void k_router_gemm(const float *s32, const float *router,
+                                                             int T, float *logits);
+#define HY3X_ROUTER_EXTERN(TMAX, MT, ME, TG, KC, R)                                             \
+  extern template __global__ void k_router_gemm<MT, ME, TG, 8, KC, R>(const float *, const float *, \
+                                                                      int, float *);
+HY3X_ROUTER_SHAPES(HY3X_ROUTER_EXTERN)
+#undef HY3X_ROUTER_EXTERN
 __global__ void k_topk(const float *logits, const float *bias, int has_bias, int K, float scale,
                        int T, int32_t *ids, float *wpre, float *wout, uint32_t *bits, int wt,
                        uint8_t *ranks);

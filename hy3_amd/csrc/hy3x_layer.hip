@@ -160,17 +160,6 @@ static int dalloc(P **p, size_t bytes) {
 // Up to this many tokens the router runs as one wave per (expert, token);
 // above it as RMSNorm + LDS-tiled GEMM + per-token top-K.
 constexpr int kSmallRouterT = 8;
-// Router GEMM tile classes by token count (shapes and measurements with
-// ROUTER_*_TINY ... XXL): TINY up to kTinyRouterT tokens, MID up to
-// kMidRouterT, LARGE up to kLargeRouterT, XL up to kXLRouterT, XXL above.
-#ifndef HY3X_ROUTER_CLASS_T
-#define HY3X_ROUTER_CLASS_T 64, 256, 1536, 2560
-#endif
-constexpr int kRouterClassT[4] = {HY3X_ROUTER_CLASS_T};
-constexpr int kTinyRouterT = kRouterClassT[0];
-constexpr int kMidRouterT = kRouterClassT[1];
-constexpr int kLargeRouterT = kRouterClassT[2];
-constexpr int kXLRouterT = kRouterClassT[3];
 // From this many tokens the experts run as MFMA grouped GEMMs. Measured on MI355X the
 // MFMA tiles beat the wavefront-reduction GEMV tiles at every T >= 2 (T=2: 51 vs 66 us,
 // T=32: 442 vs 550 us for gate/up + down), so the GEMV tiles only run when selected
@@ -538,20 +527,13 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
         k_rmsnorm<<<T, 256, 0, st>>>(x, c.xadd, L->norm_w, mf ? nullptr : S.s16, S.s32,
                                      mf ? S.s16m : nullptr, S.ssum, T, S.bits, S.wt,
                                      c.r_in);
-#define HY3X_LAUNCH_ROUTER(NAME)                                                           \
-  HY3X_ROUTER_GEMM(NAME)<<<dim3((T + 4 * ROUTER_MT_##NAME - 1) / (4 * ROUTER_MT_##NAME),     \
-                                E / (8 * ROUTER_ME_##NAME)),                                  \
-                           256, 0, st>>>(S.s32, L->router, T, S.logits)
-        if (T <= kTinyRouterT)
-          HY3X_LAUNCH_ROUTER(TINY);
-        else if (T <= kMidRouterT)
-          HY3X_LAUNCH_ROUTER(MID);
-        else if (T <= kLargeRouterT)
-          HY3X_LAUNCH_ROUTER(LARGE);
-        else if (T <= kXLRouterT)
-          HY3X_LAUNCH_ROUTER(XL);
-        else
-          HY3X_LAUNCH_ROUTER(XXL);
+#define HY3X_LAUNCH_ROUTER(TMAX, MT, ME, TG, KC, R)                                        \
+  if (T <= TMAX)                                                                           \
+    k_router_gemm<MT, ME, TG, 8, KC, R>                                                    \
+        <<<dim3((T + MT * TG - 1) / (MT * TG), E / (8 * ME)), 64 * TG, 0, st>>>(           \
+            S.s32, L->router, T, S.logits);                                                \
+  else
+        HY3X_ROUTER_SHAPES(HY3X_LAUNCH_ROUTER) {}
 #undef HY3X_LAUNCH_ROUTER
       }
       if (T <= ROUTE_SMALL_T) {

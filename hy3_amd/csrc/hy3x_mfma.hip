@@ -2,7 +2,7 @@
 //
 // A work tile is one expert, a slice of its weight matrix -- 16 WAVES
 // rows of gate and of up, or 32 WAVES rows of down (each wave 16 or
-// 2 x 16 rows) -- and up to TOKENS (32 or 64) of its tokens (the dispatch
+// 2 x 16 rows) -- and up to TOKENS (8, 32 or 64) of its tokens (the dispatch
 // tile list with NT = TOKENS), in 16-token MFMA column groups (NTT of them).
 //
 // Per Q4_K block column (256 of K):

@@ -104,18 +104,22 @@ __global__ __launch_bounds__(256) void k_rmsnorm(const float *__restrict__ x,
 // chunk is large (few blocks run at small T, so each K step's load latency is
 // paid in sequence: the fewer steps, the better).
 template <int MT, int ME, int TG, int EG, int KC, int R>
-__global__ __launch_bounds__(256) void k_router_gemm(const float *__restrict__ s32,
+__global__ __launch_bounds__(8 * TG * EG) void k_router_gemm(const float *__restrict__ s32,
                                                      const float *__restrict__ router, int T,
                                                      float *__restrict__ logits) {
-  static_assert(8 * TG * EG == 256, "256 threads");
+  constexpr int NTH = 8 * TG * EG;  // threads
+  static_assert(NTH == 256 || NTH == 512, "block size");
   static_assert(D % KC == 0 && KC % 8 == 0, "K chunks");
   constexpr int NCH = D / KC;
   static_assert(R >= 1 && NCH % R == 0, "whole rounds of the fetch ring");
   constexpr int TT = MT * TG, TE = ME * EG;
   constexpr int SP = TT + 4, WP = TE + 4;        // padded LDS rows (floats)
-  constexpr int NS = TT * KC / 4 / 256, NW = TE * KC / 4 / 256;  // float4 per thread
-  static_assert(NS >= 1 && NW >= 1, "staging split");
+  constexpr int NS = TT * KC / 4 / NTH, NW = TE * KC / 4 / NTH;  // float4 per thread
+  static_assert(NS * NTH * 4 == TT * KC && NW * NTH * 4 == TE * KC, "staging split");
   __shared__ float sl[2][KC][SP], wl[2][KC][WP];
+  // steps whose LDS reads are in flight together (T = 75: 28.5 us with 4, 26.0 with 8;
+  // from 12 outputs a thread 8 loses to the registers: T = 2048 113 -> 201 us)
+  constexpr int UN = MT * ME <= 4 ? 8 : 4;
   const int t0 = blockIdx.x * TT, e0 = blockIdx.y * TE;
   const int tid = threadIdx.x, v = tid & 7, mt = tid >> 3, tg = mt % TG, eg = mt / TG;
   // a register ring of R chunks in flight (the loop is unrolled by R so that
@@ -127,19 +131,19 @@ __global__ __launch_bounds__(256) void k_router_gemm(const float *__restrict__ s
   auto fetch = [&](int k0, float4(&sd)[NS], float4(&wd)[NW]) {
 #pragma unroll
     for (int u = 0; u < NS; u++) {
-      const int q = tid + 256 * u, r = q % TT, c = q / TT, tt = t0 + r;
+      const int q = tid + NTH * u, r = q % TT, c = q / TT, tt = t0 + r;
       sd[u] = reinterpret_cast<const float4 *>(s32 + (size_t)(tt < T ? tt : T - 1) * D + k0)[c];
     }
 #pragma unroll
     for (int u = 0; u < NW; u++) {
-      const int q = tid + 256 * u, r = q % TE, c = q / TE;
+      const int q = tid + NTH * u, r = q % TE, c = q / TE;
       wd[u] = reinterpret_cast<const float4 *>(router + (size_t)(e0 + r) * D + k0)[c];
     }
   };
   auto stage = [&](int buf, const float4(&sd)[NS], const float4(&wd)[NW]) {
 #pragma unroll
     for (int u = 0; u < NS; u++) {  // neighbouring lanes write neighbouring words
-      const int q = tid + 256 * u, r = q % TT, c = q / TT;
+      const int q = tid + NTH * u, r = q % TT, c = q / TT;
       const bool in = t0 + r < T;
       sl[buf][4 * c + 0][r] = in ? sd[u].x : 0.0f;
       sl[buf][4 * c + 1][r] = in ? sd[u].y : 0.0f;
@@ -148,7 +152,7 @@ __global__ __launch_bounds__(256) void k_router_gemm(const float *__restrict__ s
     }
 #pragma unroll
     for (int u = 0; u < NW; u++) {
-      const int q = tid + 256 * u, r = q % TE, c = q / TE;
+      const int q = tid + NTH * u, r = q % TE, c = q / TE;
       wl[buf][4 * c + 0][r] = wd[u].x;
       wl[buf][4 * c + 1][r] = wd[u].y;
       wl[buf][4 * c + 2][r] = wd[u].z;
@@ -169,7 +173,7 @@ __global__ __launch_bounds__(256) void k_router_gemm(const float *__restrict__ s
       stage(buf, sn[r], wn[r]);
       __syncthreads();  // buf staged; the other buffer is no longer read
       fetch((it + R < NCH ? it + R : NCH - 1) * KC, sn[r], wn[r]);
-#pragma unroll 4
+#pragma unroll UN
       for (int ii = 0; ii < KC / 8; ii++) {
         const int k = 8 * ii + v;
         float sv[MT], wv[ME];
@@ -193,11 +197,10 @@ __global__ __launch_bounds__(256) void k_router_gemm(const float *__restrict__ s
       if (v == 0 && tt < T) logits[(size_t)tt * E + ee] = lg;
     }
 }
-template __global__ void HY3X_ROUTER_GEMM(TINY)(const float *, const float *, int, float *);
-template __global__ void HY3X_ROUTER_GEMM(MID)(const float *, const float *, int, float *);
-template __global__ void HY3X_ROUTER_GEMM(LARGE)(const float *, const float *, int, float *);
-template __global__ void HY3X_ROUTER_GEMM(XL)(const float *, const float *, int, float *);
-template __global__ void HY3X_ROUTER_GEMM(XXL)(const float *, const float *, int, float *);
+#define HY3X_ROUTER_INSTANCE(TMAX, MT, ME, TG, KC, R) \
+  template __global__ void k_router_gemm<MT, ME, TG, 8, KC, R>(const float *, const float *, int, float *);
+HY3X_ROUTER_SHAPES(HY3X_ROUTER_INSTANCE)
+#undef HY3X_ROUTER_INSTANCE
 
 // Routing of token t in one wave: sigmoid and score of the 192 logits (expert
 // lane + 64 m in slot m), the top-K in registers (topk_wave_fast, or
@@ -344,8 +347,7 @@ __global__ __launch_bounds__(64 * ROUTE_SMALL_T) void k_route_small(
 // Block E also writes the tile counts, the per-expert counts and the stats.
 __global__ __launch_bounds__(256) void k_dispatch_list(
     const uint8_t *__restrict__ ranks, int T, int K, int NT, const uint32_t *__restrict__ bits,
-    int wt, int32_t *__restrict__ list,
-    int4 *__restrict__ tiles, int32_t *__restrict__ n_tiles, int max_tiles, int NT2,
+    int wt, int32_t *__restrict__ list, int4 *__restrict__ tiles, int32_t *__restrict__ n_tiles, int max_tiles, int NT2,
     int4 *__restrict__ tiles2, int32_t *__restrict__ n_tiles2,
     int32_t *__restrict__ counts_out, unsigned long long *__restrict__ stats) {
   __shared__ int tmp[8], off_l, toff_l, ce_l;

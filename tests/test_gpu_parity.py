@@ -165,6 +165,14 @@ def test_routing_at_router_tile_boundaries(torch, layer, cpu, T, K):
     assert np.array_equal(w.view(np.uint32), r["w"].view(np.uint32))
 
 
+@pytest.mark.parametrize("T,K", [(9, 8), (40, 8), (41, 8), (80, 8), (81, 5), (168, 8), (169, 8),
+                                 (336, 8), (337, 1), (672, 8), (673, 8), (1344, 8), (1345, 7)])
+def test_routing_at_router_shape_boundaries(torch, layer, cpu, T, K):
+    """Both sides of the router GEMM shapes' boundaries (the last tokens of a
+    block tile beyond T at the odd ones): routing bit-exact."""
+    test_routing_at_router_tile_boundaries(torch, layer, cpu, T, K)
+
+
 @pytest.mark.parametrize("T", [319, 320, 1151, 1152])
 def test_default_path_thresholds(torch, layer, cpu, T):
     """At both sides of the default path's changes of tile shape (narrow to
