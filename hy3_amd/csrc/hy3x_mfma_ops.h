@@ -118,9 +118,9 @@ __device__ __forceinline__ h8_t mins_operand(uint32_t hx, uint32_t mw, uint32_t 
 // of the launch: with Q8 weights they take twice as long as a routed expert's,
 // and at the end of one XCD's work they were the launch's tail (8 tokens, Q8:
 // gate/up 95.7 us and down 46.8, first and spread 83.4 and 40.4; 20: 146.8 and
-// 86.5, 139.7 and 69.4). The rest: consecutive items on one XCD,
-// so that the row tiles of one expert tile share its activations in that XCD's
-// L2, and consecutive token tiles of one expert share its weights.
+// 86.5, 139.7 and 69.4). The rest: consecutive items on one XCD, so that the row
+// tiles of one expert tile share its activations in that XCD's L2, and
+// consecutive token tiles of one expert share its weights.
 __device__ __forceinline__ int xcd_remap(int bid, int nblocks, int shared) {
   const int s8 = shared & ~7;
   if (bid < s8) return bid;

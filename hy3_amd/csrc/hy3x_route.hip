@@ -340,8 +340,9 @@ __global__ __launch_bounds__(64 * ROUTE_SMALL_T) void k_route_small(
 }
 
 // Dispatch lists from the bitmaps k_topk marked, one block per expert (E + 1
-// blocks, the last is the shared expert): list offset and first tile from exclusive scans of all counts, the expert's
-// tiles, and its slots in token order from its bitmap (popcount prefix sums).
+// blocks, the last is the shared expert): list offset and first tile from
+// exclusive scans of all counts, the expert's tiles, and its slots in token order
+// from its bitmap (popcount prefix sums).
 // NT2 != 0: a second tile list over the same slots, of at most NT2 tokens per
 // tile (the two lists' offsets are then scanned packed: fewer than 32768 tiles).
 // Block E also writes the tile counts, the per-expert counts and the stats.
