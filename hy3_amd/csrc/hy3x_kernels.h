@@ -159,8 +159,9 @@ extern template __global__ void k_moe_big<false>(const uint8_t *, const uint8_t 
                                                  int, int, __half *, float *);
 }  // namespace mfma_big
 // The down GEMM for few tokens per expert (hy3x_mfma_few.hip): work tiles of
-// 16 FEW_WAVES rows and up to FEW_TOKENS tokens.
-constexpr int FEW_TOKENS = 4, FEW_WAVES = 4;
+// 16 FEW_WAVES rows and up to FEW_TOKENS tokens (up to FEW_ROWS: their h rows
+// whole in LDS).
+constexpr int FEW_TOKENS = 16, FEW_ROWS = 4, FEW_WAVES = 4;
 __global__ void k_down_few(const uint8_t *wq, const uint8_t *wsh, const __half *act,
                            const __half *act_sum, const int32_t *list, const int4 *tiles,
                            const int32_t *n_tiles, int T, float *out);

@@ -173,10 +173,13 @@ constexpr int kMfmaMinT = 2;
 // vs 30.2, 3: 49.5 vs 45.0, 4: 53.7 vs 48.8, 5: 58.0 vs 62.6, 6: 66.6 vs 70.5, 8:
 // 80.1 vs 75-83.
 constexpr int kTinyMinRowTiles = 512, kTinyMaxRowTiles = 800;
-// Up to this many tokens the down GEMM keeps whole rows in registers
-// (k_down_few); above it the MFMA tiles' reuse of the dequantised weights wins.
-// Down launch us, narrow tiles vs whole rows: 2 tokens 19.4 vs 15.2, 8: 43.7 vs
-// 37.2, 16: 71.1 vs 57.7, 32: 91.0 vs 81.0, 48: 106.8 vs 101.7, 64: 116.1 vs 121.5.
+// Up to this many tokens the down GEMM keeps whole rows in registers (k_down_few):
+// three tiles of 16 tokens of an expert at most. Down launch us, K = 8, weights from
+// HBM, narrow tiles vs whole rows, tokens evenly spread: 2 tokens 21.7 vs 18.9, 8:
+// 48.5 vs 39.7, 32: 94.5 vs 81.9, 48: 107.6 vs 97.1, 64: 115.5 vs 109.0, 96: 126.9 vs
+// 124.2; every token on the same eight experts: 8: 15.3 vs 15.4, 32: 19.0 vs 20.6, 48:
+// 22.2 vs 26.0, but 56: 24.5 vs 30.4, 64: 24.8 vs 30.6. The dispatch is not known
+// on the host, so the line lies where a fourth tile would begin.
 constexpr int kDownFewMaxT = 48;
 // From this many tokens the MFMA GEMMs use the wide tile shape (64 tokens, 8 waves).
 // Measured on MI355X (ms per layer, narrow vs wide): 32 tokens 0.32 vs 0.37,
