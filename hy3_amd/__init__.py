@@ -66,6 +66,7 @@ _SIGS = {
     "hy3x_layer_set_path": (I32, [P, I32]),
     "hy3x_layer_set_rms_scale": (I32, [P, P, I32]),
     "hy3x_layer_last_path": (I32, [P, ctypes.POINTER(ctypes.c_int)]),
+    "hy3x_layer_last_kernel": (I32, [P, I32, ctypes.POINTER(ctypes.c_char_p)]),
     "hy3x_layer_time_stage": (I32, [P, I32, I32, P, ctypes.POINTER(ctypes.c_float)]),
     "hy3x_layers_time_stage": (I32, [ctypes.POINTER(P), I32, I32, I32, P,
                                      ctypes.POINTER(ctypes.c_float)]),
@@ -246,7 +247,7 @@ class MoELayer:
     def synth_shared_q8_0(self, seed, layer_index=0):
         _check(lib().hy3x_synth_shared_q8_0(self._h, seed, layer_index))
 
-    path = 0  # 0 auto, 1 GEMV, 2 MFMA, 3 MFMA narrow, 4 MFMA wide (hy3x_layer_set_path)
+    path = 0  # 0 auto, 1 GEMV, 2 MFMA, 3 / 4 / 5 MFMA narrow / wide / 128-token (hy3x_layer_set_path)
 
     def set_path(self, path):
         _check(lib().hy3x_layer_set_path(self._h, path))
@@ -254,10 +255,16 @@ class MoELayer:
 
     def last_path(self):
         """Expert path of the last forward: 0 decode kernels, 1 GEMV tiles,
-        3 / 4 MFMA narrow / wide tiles."""
+        3 / 4 / 5 MFMA narrow / wide / 128-token tiles."""
         v = ctypes.c_int()
         _check(lib().hy3x_layer_last_path(self._h, ctypes.byref(v)))
         return v.value
+
+    def last_kernel(self, stage):
+        """Name of the kernel the last forward ran in stage "gateup" or "down"."""
+        v = ctypes.c_char_p()
+        _check(lib().hy3x_layer_last_kernel(self._h, self.STAGES.index(stage), ctypes.byref(v)))
+        return v.value.decode()
 
     def set_rms_scale(self, r=None):
         """Substitute the per-token RMSNorm scale (None: compute it again)."""

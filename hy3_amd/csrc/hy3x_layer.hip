@@ -499,6 +499,30 @@ int hy3x_layer_last_path(const hy3x_layer *L, int *path) {
   return HY3X_OK;
 }
 
+int hy3x_layer_last_kernel(const hy3x_layer *L, int stage, const char **name) {
+  if (!L || !name) return fail(HY3X_E_ARG, "NULL argument");
+  if (stage != HY3X_STAGE_GATEUP && stage != HY3X_STAGE_DOWN)
+    return fail(HY3X_E_ARG, "stage %d is neither gate/up nor down", stage);
+  if (!L->last_T) return fail(HY3X_E_STATE, "no forward yet");
+  const auto &c = L->cur;
+  const bool gu = stage == HY3X_STAGE_GATEUP;
+  if (c.mode == Mode::DECODE)
+    *name = gu ? "k_gateup_decode" : "k_down_decode";
+  else if (c.mode == Mode::GEMV)
+    *name = gu ? "k_gateup_gemv<4>" : "k_down_gemv<4>";
+  else if (gu && c.tiny)
+    *name = "mfma_tiny::k_moe_mfma<true>";
+  else if (!gu && c.few)
+    *name = "k_down_few";
+  else if (c.big)
+    *name = gu ? "mfma_big::k_moe_big<true>" : "mfma_big::k_moe_big<false>";
+  else if (c.wide)
+    *name = gu ? "mfma_wide::k_moe_mfma<true>" : "mfma_wide::k_moe_mfma<false>";
+  else
+    *name = gu ? "mfma_narrow::k_moe_mfma<true>" : "mfma_narrow::k_moe_mfma<false>";
+  return HY3X_OK;
+}
+
 // Kernels of one stage for the forward described by L->cur (shared by the
 // forward and the kernel replay used for timing).
 static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {

@@ -251,10 +251,15 @@ int hy3x_layer_set_path(hy3x_layer *layer, int path);
 
 /* Which expert path the last forward ran: 0 = the fused single-token decode
  * kernels, 1 = wavefront-GEMV tiles, 3 = MFMA with the narrow tile shape (by
- * itself, path 0, with variants of it for few tokens that give the same bits),
- * 4 = MFMA with the wide one, 5 = MFMA with 128-token tiles (diagnostics and benchmarks: the kernel whose
- * roofline a benchmark reports). */
+ * itself, path 0, with variants of it for few tokens that give the same bits:
+ * hy3x_layer_last_kernel tells them apart), 4 = MFMA with the wide one, 5 = MFMA
+ * with 128-token tiles. */
 int hy3x_layer_last_path(const hy3x_layer *layer, int *path);
+
+/* Name of the expert GEMM or GEMV kernel the last forward ran in stage
+ * HY3X_STAGE_GATEUP or HY3X_STAGE_DOWN (a constant string; diagnostics and
+ * benchmarks: the kernel whose roofline a benchmark reports). */
+int hy3x_layer_last_kernel(const hy3x_layer *layer, int stage, const char **name);
 
 /* ---- synthetic inputs (test / benchmark data, not part of the MoE path) ----
  * Device-side generator + Q4_K quantiser for the seeded synthetic layers the

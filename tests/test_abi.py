@@ -52,6 +52,7 @@ def test_argument_errors_are_codes():
     assert lib.hy3x_layer_forward(None, None, 1, 8, 2.826, None) == -1
     assert lib.hy3x_layer_set_router(None, None, None, None) == -1
     assert lib.hy3x_layer_set_expert_q4k(None, 0, None, None, None, 0) == -1
+    assert lib.hy3x_layer_last_kernel(None, 2, None) == -1
     assert lib.hy3x_layer_destroy(None) == 0
     assert lib.hy3x_synth_quantize_q4k(None, None, 100, None) == -1
 

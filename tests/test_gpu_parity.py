@@ -173,6 +173,30 @@ def test_routing_at_router_shape_boundaries(torch, layer, cpu, T, K):
     test_routing_at_router_tile_boundaries(torch, layer, cpu, T, K)
 
 
+@pytest.mark.parametrize("T,K,path,gateup,down", [
+    (1, 8, 0, "k_gateup_decode", "k_down_decode"),
+    (2, 8, 0, "mfma_narrow::k_moe_mfma<true>", "k_down_few"),
+    (3, 8, 0, "mfma_tiny::k_moe_mfma<true>", "k_down_few"),
+    (8, 4, 0, "mfma_tiny::k_moe_mfma<true>", "k_down_few"),
+    (8, 8, 1, "k_gateup_gemv<4>", "k_down_gemv<4>"),
+    (48, 8, 0, "mfma_narrow::k_moe_mfma<true>", "k_down_few"),
+    (48, 8, 3, "mfma_narrow::k_moe_mfma<true>", "mfma_narrow::k_moe_mfma<false>"),
+    (49, 8, 0, "mfma_narrow::k_moe_mfma<true>", "mfma_narrow::k_moe_mfma<false>"),
+    (320, 8, 0, "mfma_wide::k_moe_mfma<true>", "mfma_wide::k_moe_mfma<false>"),
+    (16, 8, 5, "mfma_big::k_moe_big<true>", "mfma_big::k_moe_big<false>")])
+def test_last_kernel_names_what_ran(torch, layer, T, K, path, gateup, down):
+    """hy3x_layer_last_kernel names the kernel of either expert stage, the
+    few-token variants included (hy3x_layer_last_path calls them narrow)."""
+    layer.set_path(path)
+    try:
+        run(torch, layer, C.inputs(0xCB, T), K)
+        assert (layer.last_kernel("gateup"), layer.last_kernel("down")) == (gateup, down)
+        with pytest.raises(H.HY3XError):
+            layer.last_kernel("router")
+    finally:
+        layer.set_path(0)
+
+
 @pytest.mark.parametrize("T", [319, 320, 1151, 1152])
 def test_default_path_thresholds(torch, layer, cpu, T):
     """At both sides of the default path's changes of tile shape (narrow to
