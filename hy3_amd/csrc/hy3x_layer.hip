@@ -166,12 +166,17 @@ constexpr int kSmallRouterT = 8;
 // explicitly (hy3x_layer_set_path 1); T = 1 keeps the fused decode kernels.
 constexpr int kMfmaMinT = 2;
 // Up to 8 tokens, gate/up runs in the 8-token shape (mfma_tiny: three workgroups
-// per CU, 768 in all, against the narrow shape's 512) where the routed experts'
-// row tiles, if no two tokens share one, overfill one round of the narrow shape
-// but about fill one of these: a second round for a few of them costs a whole
-// item's 16 columns. Gate/up us, narrow vs 8-token shape, K = 8: 2 tokens 29.7
-// vs 30.2, 3: 49.5 vs 45.0, 4: 53.7 vs 48.8, 5: 58.0 vs 62.6, 6: 66.6 vs 70.5, 8:
-// 80.1 vs 75-83.
+// per CU, 768 in all, against the narrow shape's 512) where the row tiles of the
+// experts, if no two tokens share a routed one, overfill one round of the narrow
+// shape and at most just overfill one of these (some tokens share experts): a
+// second round for a few of them costs a whole item's 16 columns. Gate/up us,
+// weights from HBM, narrow vs 8-token shape, evenly spread: K = 8, 3 tokens 49.0 vs
+// 44.7, 4: 53.0 vs 46.5 (792 row tiles); K = 6, 5 tokens 52.4 vs 46.1; K = 4, 6: 42.6
+// vs 39.7, 8: 52.6 vs 46.7; K = 3, 8: 40.3 vs 38.4; every token on the same experts
+// equal. Outside: K = 8, 2 tokens 29.7 vs 30.2, 5: 58.0 vs 62.6, 6: 66.6 vs 70.5. Not
+// with a Q8 shared expert: its items take twice as long and set the end of the
+// launch, three to a CU later than two (K = 8, 3 tokens 49.6 vs 52.9, 4: 54.3 vs 56.3;
+// K = 4, 8: 51.8 vs 54.4).
 constexpr int kTinyMinRowTiles = 512, kTinyMaxRowTiles = 800;
 // Up to this many tokens the down GEMM keeps whole rows in registers (k_down_few):
 // three tiles of 16 tokens of an expert at most. Down launch us, K = 8, weights from
@@ -593,8 +598,7 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
       else if (c.mode == Mode::MFMA && c.tiny)
         mfma_tiny::k_moe_mfma<true>
             <<<mt * (F / mfma_tiny::ROWS_GU), 64 * mfma_tiny::WAVES, 0, st>>>(
-                L->wq, L->shared_q8 ? L->wsh : nullptr, S.s16m, S.ssum, S.list, S.tiles,
-                S.n_tiles, T, K, S.h16m, nullptr);
+                L->wq, nullptr, S.s16m, S.ssum, S.list, S.tiles, S.n_tiles, T, K, S.h16m, nullptr);
       else if (c.mode == Mode::MFMA && c.big)
         mfma_big::k_moe_big<true><<<(mt + XCD_TILE_RR_MARGIN) * (F / (16 * BIG_WAVES)), 64 * BIG_WAVES, 0, st>>>(
             L->wq, L->shared_q8 ? L->wsh : nullptr, S.s16m, S.ssum, S.list, S.tiles, S.n_tiles, T, K, S.h16m, nullptr);
@@ -716,7 +720,7 @@ static int forward_impl(hy3x_layer *L, const Scratch *sc, const hy3x_layer **own
            (L->path == 4 || (L->path != 3 && T >= kMfmaWideMinT));
   const bool by_t = c.mode == Mode::MFMA && (L->path == 0 || L->path == 2);
   const int row_tiles = (T * K + 1) * (F / mfma_tiny::ROWS_GU);
-  c.tiny = by_t && T <= mfma_tiny::TOKENS && row_tiles > kTinyMinRowTiles &&
+  c.tiny = by_t && !L->shared_q8 && T <= mfma_tiny::TOKENS && row_tiles > kTinyMinRowTiles &&
            row_tiles <= kTinyMaxRowTiles;
   c.few = by_t && T <= kDownFewMaxT;
   // tokens per work tile

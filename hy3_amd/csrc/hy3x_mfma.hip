@@ -431,7 +431,7 @@ __device__ __forceinline__ void mfma_tile(const uint8_t *__restrict__ wq,
 // permute, minus 1152) and each block's MFMA result is scaled by its d in
 // fp32: acc += d_b * (x_b . q_b) -- sum d*q*x as mul_mat_f32 case 8
 // (hy3.c:1098-1120).
-constexpr int B8_DMA = MT_TOK < 16 ? 1 : MT_TOK * 16 / 64 / MT_WAVES;  // activation copies per wave
+constexpr int B8_DMA = MT_TOK * 16 / 64 / MT_WAVES;  // activation copies per wave
 
 template <bool GATEUP, int NTT>
 struct TileStateQ8 {
@@ -493,7 +493,7 @@ __device__ __forceinline__ void mfma_step_q8(TileStateQ8<GATEUP, NTT> &st, int k
   for (int t = 0; t < NTT; t++)
 #pragma unroll
     for (int b = 0; b < 4; b++)
-      x[t][b] = __builtin_bit_cast(h8_t, bt[16 * tok_row(16 * t + lr) + ((4 * b + g) ^ swz(lr))]);
+      x[t][b] = __builtin_bit_cast(h8_t, bt[16 * (16 * t + lr) + ((4 * b + g) ^ lr)]);
   const f4_t zero4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int b = 0; b < 4; b++) {
@@ -538,7 +538,7 @@ __device__ __forceinline__ void mfma_tile_q8(const uint8_t *__restrict__ wsh,
   st.bbase = reinterpret_cast<const uint8_t *>(act);
 #pragma unroll
   for (int j = 0; j < B8_DMA; j++) {
-    const int q = 64 * (B8_DMA * wave + j) + lane, r = tok_row(q >> 4);
+    const int q = 64 * (B8_DMA * wave + j) + lane, r = q >> 4;
     const int ar = t_arow[r] >= 0 ? t_arow[r] : arow0;
     st.boff[j] = (uint32_t)(2 * (ar * KD + 8 * ((q & 15) ^ (r & 15))));
   }
@@ -592,22 +592,24 @@ __global__ __launch_bounds__(MT_THREADS) void k_moe_mfma(
     t_arow[tid] = s < 0 ? -1 : (GATEUP ? (s < T * K ? s / K : s - T * K) : s);
   }
   __syncthreads();
-  if (wsh && e == E) {
-    if constexpr (MT_TOK > 32) {
-      if (n > 48) {
-        mfma_tile_q8<GATEUP, 4>(wsh, act, n, rt, h16m, out);
-        return;
+  if constexpr (MT_TOK > 16) {  // the 8-token shape runs with a Q4_K shared expert only
+    if (wsh && e == E) {
+      if constexpr (MT_TOK > 32) {
+        if (n > 48) {
+          mfma_tile_q8<GATEUP, 4>(wsh, act, n, rt, h16m, out);
+          return;
+        }
+        if (n > 32) {
+          mfma_tile_q8<GATEUP, 3>(wsh, act, n, rt, h16m, out);
+          return;
+        }
       }
-      if (n > 32) {
-        mfma_tile_q8<GATEUP, 3>(wsh, act, n, rt, h16m, out);
-        return;
-      }
+      if (n > 16)
+        mfma_tile_q8<GATEUP, 2>(wsh, act, n, rt, h16m, out);
+      else
+        mfma_tile_q8<GATEUP, 1>(wsh, act, n, rt, h16m, out);
+      return;
     }
-    if (MT_TOK > 16 && n > 16)
-      mfma_tile_q8<GATEUP, (MT_TOK > 16 ? 2 : 1)>(wsh, act, n, rt, h16m, out);
-    else
-      mfma_tile_q8<GATEUP, 1>(wsh, act, n, rt, h16m, out);
-    return;
   }
   if constexpr (MT_TOK > 32) {
     if (n > 48) {

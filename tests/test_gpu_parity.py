@@ -852,6 +852,16 @@ def test_q8_shared_few_token_kernels_equal_narrow_tiles(torch, q8_layer, T):
     assert np.array_equal(y0.view(np.uint32), y3.view(np.uint32))
 
 
+@pytest.mark.parametrize("T,K", [(3, 8), (4, 8), (8, 4)])
+def test_q8_shared_keeps_narrow_gateup(torch, q8_layer, T, K):
+    """With the Q8_0 shared expert the 8-token gate/up shape, which its long
+    items slow down, is not chosen; a Q4_K shared expert gets it
+    (test_last_kernel_names_what_ran)."""
+    run(torch, q8_layer, C.inputs(0xCC, T), K)
+    assert q8_layer.last_kernel("gateup") == "mfma_narrow::k_moe_mfma<true>"
+    assert q8_layer.last_kernel("down") == "k_down_few"
+
+
 def test_q8_shared_reference_tokens(torch, q8_layer):
     """hy3.c's forward_layer_moe with the Q8_0 shared expert on three config-1
     tokens (moe_q8.npz), through the batched (MFMA) path."""
