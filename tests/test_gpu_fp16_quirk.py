@@ -133,13 +133,20 @@ def test_quirk_blocks_differ_from_ieee():
     assert (a[0::2] != b[0::2]).any(axis=1).all()  # every patched block decodes differently
 
 
-@pytest.mark.parametrize("T,path", [(1, 0), (8, 1), (8, 3), (8, 4), (8, 5), (1, 2)])
+@pytest.mark.parametrize("T,path", [(1, 0), (8, 1), (8, 3), (8, 4), (8, 5), (1, 2), (3, 0), (4, 0),
+                                    (8, 0)])
 def test_quirk_blocks_on_every_path(torch, quirk_layer, T, path):
     """Decode kernels (T = 1), GEMV tiles, narrow, wide and 128-token MFMA
-    tiles, and MFMA at T = 1: routing bit-exact, output within TOL of the
-    oracle."""
+    tiles, MFMA at T = 1, and the kernels that serve few tokens by default (3
+    and 4: the 8-token gate/up shape; all three: the whole-row down GEMM, at 8
+    with a tile of more than four tokens): routing bit-exact, output within TOL
+    of the oracle."""
     L, cpu, x = quirk_layer
     run_path(torch, L, cpu, x[:T], path)
+    if path == 0 and T > 1:
+        assert L.last_kernel("down") == "k_down_few"
+        tiny = L.last_kernel("gateup") == "mfma_tiny::k_moe_mfma<true>"
+        assert tiny == (T in (3, 4))
 
 
 @pytest.mark.parametrize("path", [4, 5])
@@ -150,11 +157,12 @@ def test_quirk_blocks_130_tokens(torch, quirk_layer_130, path):
     run_path(torch, L, cpu, x, path)
 
 
-@pytest.mark.parametrize("T,path", [(1, 0), (8, 3), (8, 4), (8, 5)])
+@pytest.mark.parametrize("T,path", [(1, 0), (8, 3), (8, 4), (8, 5), (3, 0), (8, 0)])
 def test_quirk_blocks_with_q8_shared(torch, quirk_layer, T, path):
     """The routed experts' quirk blocks on the kernels' Q8_0-shared variants
-    (hy3's real-checkpoint shared expert: the decode kernels and the narrow,
-    wide and 128-token MFMA tiles with mfma_tile_q8): routing bit-exact, output
+    (hy3's real-checkpoint shared expert: the decode kernels, the narrow, wide
+    and 128-token MFMA tiles with mfma_tile_q8, and the whole-row down GEMM of
+    the default path): routing bit-exact, output
     within TOL of the oracle holding the same Q8_0 shared expert."""
     L, cpu, x = quirk_layer
     q8 = tuple(O.gen_matrix_q8(C.WEIGHT_SEED, 0, k, E) for k in (O.T_GATE, O.T_UP, O.T_DOWN))
