@@ -206,7 +206,7 @@ __device__ __forceinline__ void issue_a(const State &st, int ka) {
   const uint8_t *ab = st.abase + (size_t)ka * QB;
 #pragma unroll
   for (int j = 0; j < A_DMA; j++)
-    if (j < A_DMA - 1 || st.a_last) dma16_stream(ab, st.aoff[j], lds_addr(dst + 64 * j));
+    if (j < A_DMA - 1 || st.a_last) dma16_s(ab, st.aoff[j], lds_addr(dst + 64 * j));
 }
 
 // One block column kb. Its copies were issued one (activations) and A_AHEAD

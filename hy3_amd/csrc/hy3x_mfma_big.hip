@@ -100,7 +100,7 @@ __device__ __forceinline__ void issue_w(const State<GATEUP, NTT> &st, int kb) {
   const uint8_t *ab = st.abase + (size_t)kb * QB;
 #pragma unroll
   for (int j = 0; j < A_DMA; j++)
-    if (j < A_DMA - 1 || st.a_last) dma16_stream(ab, st.aoff[j], lds_addr(dst + 64 * j));
+    if (j < A_DMA - 1 || st.a_last) dma16_s(ab, st.aoff[j], lds_addr(dst + 64 * j));
 }
 template <bool GATEUP, int NTT>
 __device__ __forceinline__ void issue_x(const State<GATEUP, NTT> &st, int s) {

@@ -14,14 +14,6 @@ typedef float f4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t u4_t __attribute__((ext_vector_type(4)));  // 16 bytes as a native vector
 typedef uint32_t u2_t __attribute__((ext_vector_type(2)));
 
-// dma16_stream is the weight copy, with the default cache policy (a
-// non-temporal one measured ~15% slower).
-__device__ __forceinline__ void dma16_stream(const void *sbase, uint32_t voff, uint32_t lds) {
-  asm volatile("global_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase),
-               "{m0}"(lds)
-               : "memory");
-}
-
 __device__ __forceinline__ uint32_t pk_fma_f16(uint32_t a, h2_t b, h2_t c) {
   return __builtin_bit_cast(uint32_t, __builtin_elementwise_fma(as_h2(a), b, c));
 }
