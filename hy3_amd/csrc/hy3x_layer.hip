@@ -529,8 +529,9 @@ int hy3x_layer_last_kernel(const hy3x_layer *L, int stage, const char **name) {
 }
 
 // Kernels of one stage for the forward described by L->cur (shared by the
-// forward and the kernel replay used for timing).
-static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
+// forward and the kernel replay used for timing, which passes no stats: a
+// replay is no forward).
+static void launch_stage(hy3x_layer *L, int stage, hipStream_t st, unsigned long long *stats) {
   const auto &c = L->cur;
   const Scratch &S = c.sc;
   const int T = c.T, K = c.K, mt = c.mt;
@@ -572,7 +573,7 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
         k_route_small<<<1, 64 * ROUTE_SMALL_T, 0, st>>>(
             S.logits, L->bias, L->has_bias, K, c.scale, T, c.nt, S.ids, S.wpre, S.w, S.list,
             S.tiles, S.n_tiles, mt, c.few ? FEW_TOKENS : 0, S.tiles2, S.n_tiles2, S.counts,
-            L->stats);
+            stats);
       } else {
         // one wave per token; up to 256 tokens one wave per block, so that
         // few tokens still spread over many CUs
@@ -587,14 +588,14 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st) {
         k_dispatch_list<<<E + 1, 256, 0, st>>>(S.ranks, T, K, c.nt, S.bits, S.wt,
                                                S.list, S.tiles, S.n_tiles, mt,
                                                c.few ? FEW_TOKENS : 0, S.tiles2, S.n_tiles2,
-                                               S.counts, L->stats);
+                                               S.counts, stats);
       }
       break;
     case HY3X_STAGE_GATEUP:
       if (c.mode == Mode::DECODE)
         k_gateup_decode<<<K * DEC_GU_BLOCKS, 64 * DEC_GU_WAVES, 0, st>>>(L->wq, S.s16, S.sig, S.score, K,
                                                           c.scale, S.ids, S.wpre, S.w,
-                                                          L->stats, S.h16, L->trace[1]);
+                                                          stats, S.h16, L->trace[1]);
       else if (c.mode == Mode::MFMA && c.tiny)
         mfma_tiny::k_moe_mfma<true>
             <<<mt * (F / mfma_tiny::ROWS_GU), 64 * mfma_tiny::WAVES, 0, st>>>(
@@ -733,7 +734,7 @@ static int forward_impl(hy3x_layer *L, const Scratch *sc, const hy3x_layer **own
   for (int stage = HY3X_STAGE_ROUTER; stage <= HY3X_STAGE_COMBINE; stage++) {
     if (c.mode == Mode::DECODE && (stage == HY3X_STAGE_DISPATCH || stage == HY3X_STAGE_COMBINE))
       continue;
-    launch_stage(L, stage, st);
+    launch_stage(L, stage, st, L->stats);
     record_stage(L, st, stage);
   }
   if (L->timing) L->n_timed++;
@@ -759,7 +760,7 @@ int hy3x_layers_time_stage(hy3x_layer *const *layers, int n, int stage, int reps
   EventPair ev;
   HIP_TRY(ev.create());
   HIP_TRY(hipEventRecord(ev.a, st));
-  for (int i = 0; i < reps; i++) launch_stage(layers[i % n], stage, st);
+  for (int i = 0; i < reps; i++) launch_stage(layers[i % n], stage, st, nullptr);
   HIP_TRY(hipEventRecord(ev.b, st));
   HIP_TRY(hipEventSynchronize(ev.b));
   float ms = 0.0f;

@@ -187,8 +187,8 @@ int hy3x_layer_last_routing(hy3x_layer *layer, int32_t *ids, float *wpre, float 
  * hy3x_layer_stage_times() synchronises, returns the accumulated milliseconds
  * per stage (index HY3X_STAGE_*) and the number of forwards timed, and resets
  * the accumulators. Enabling also resets. */
-#define HY3X_STAGE_ROUTER 0   /* RMSNorm + router GEMV + top-K        */
-#define HY3X_STAGE_DISPATCH 1 /* per-expert lists and work tiles      */
+#define HY3X_STAGE_ROUTER 0   /* RMSNorm + router GEMV + top-K; up to 8 tokens the lists and tiles too */
+#define HY3X_STAGE_DISPATCH 1 /* per-expert lists and work tiles (nothing up to 8 tokens) */
 #define HY3X_STAGE_GATEUP 2   /* gate/up GEMV or GEMM + SwiGLU         */
 #define HY3X_STAGE_DOWN 3     /* down GEMV or GEMM                     */
 #define HY3X_STAGE_COMBINE 4  /* weighted combine + residual           */
@@ -200,8 +200,9 @@ int hy3x_layer_stage_times(hy3x_layer *layer, float *ms, int n_stages, int *n_fo
  * forward `reps` times back to back on `stream`, bracketed by two HIP events,
  * and returns the mean microseconds per launch in *us (synchronises). Inputs
  * are those of the last forward, so the x buffer it named must still be live;
- * the down stage of a single-token forward adds its output into x again, so x
- * is modified. No reference counterpart (measurement only). */
+ * the stage that writes x (down for a single token, else combine) adds into it
+ * again. hy3x_layer_stats does not count replays. No reference counterpart
+ * (measurement only). */
 int hy3x_layer_time_stage(hy3x_layer *layer, int stage, int reps, void *stream, float *us);
 /* The same over n layers in rotation (launch i replays layers[i % n]'s stage),
  * so that with n layers whose weights together exceed the last-level cache

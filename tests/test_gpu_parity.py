@@ -197,6 +197,21 @@ def test_last_kernel_names_what_ran(torch, layer, T, K, path, gateup, down):
         layer.set_path(0)
 
 
+@pytest.mark.parametrize("T", [1, 3, 8, 9])
+def test_stage_replays_are_no_forwards(torch, layer, T):
+    """hy3x_layer_time_stage leaves the counters of hy3x_layer_stats alone, in
+    whichever stage the forward counts itself: gate/up (1 token), router (up to
+    8) or dispatch."""
+    x = torch.from_numpy(C.inputs(0xCD, T)).cuda()
+    torch.cuda.synchronize()
+    layer.stats()
+    layer.forward(x.data_ptr(), T)
+    for stage in ("router", "dispatch", "gateup"):
+        if T > 1 or stage != "dispatch":
+            layer.time_stage(stage, 3)
+    assert layer.stats()[0] == 1
+
+
 @pytest.mark.parametrize("T", [319, 320, 1151, 1152])
 def test_default_path_thresholds(torch, layer, cpu, T):
     """At both sides of the default path's changes of tile shape (narrow to
