@@ -66,9 +66,9 @@ __device__ __forceinline__ float half_sum(float v) {
 }
 
 // DPP moves (gfx9 encodings): quad_perm [1,0,3,2] / [2,3,0,1], row_half_mirror,
-// row_mirror, row_bcast:15, row_bcast:31, row_ror:8.
+// row_mirror, row_bcast:15, row_bcast:31.
 constexpr int DPP_XOR1 = 0xB1, DPP_XOR2 = 0x4E, DPP_HALF_MIRROR = 0x141, DPP_MIRROR = 0x140,
-              DPP_BCAST15 = 0x142, DPP_BCAST31 = 0x143, DPP_ROR8 = 0x128;
+              DPP_BCAST15 = 0x142, DPP_BCAST31 = 0x143;
 
 template <int CTRL, int ROW_MASK = 0xF>
 __device__ __forceinline__ float dpp(float v) {

@@ -8,8 +8,7 @@ __global__ void k_router_logits(const float *x, const float *xadd, const float *
                                 const float *router,
                                 const float *bias, int has_bias, float *logits, float *sig,
                                 float *score, __half *s16, float *s32, __half *s16m,
-                                __half *ssum, unsigned long long *trace, int T,
-                                uint32_t *bits, int wt, const float *r_in);
+                                __half *ssum, unsigned long long *trace, const float *r_in);
 __global__ void k_rmsnorm(const float *x, const float *xadd, const float *norm_w, __half *s16,
                           float *s32,
                           __half *s16m, __half *ssum, int T, uint32_t *bits, int wt,
@@ -56,12 +55,12 @@ __global__ void k_dispatch_list(const uint8_t *ranks, int T, int K, int NT, cons
                                 int32_t *n_tiles, int max_tiles, int NT2, int4 *tiles2,
                                 int32_t *n_tiles2, int32_t *counts_out,
                                 unsigned long long *stats);
-// Up to this many tokens one block routes every token and makes the dispatch
-// lists (k_route_small), in one launch where top-K, staging and dispatch were
-// three: 2 / 3 / 4 / 8 tokens 73.4 / 99.5 / 108.0 / 155.9 -> 64.4 / 90.0 / 98.3 /
-// 145.9 us per forward. It ends where the router stops running one wave per
-// (expert, token) and one wave per token still fits one block; the T > 8 router
-// stages s in k_rmsnorm and its dispatch alone takes about 4 us. tiles2: the
+// Up to this many tokens the router runs as one wave per (expert, token)
+// (k_router_logits; above as RMSNorm + LDS-tiled GEMM + per-token top-K), and one
+// block routes every token and makes the dispatch lists (k_route_small), in one
+// launch where top-K, staging and dispatch were three: 2 / 3 / 4 / 8 tokens 73.4 / 99.5 / 108.0 / 155.9 -> 64.4 / 90.0 / 98.3 /
+// 145.9 us per forward. It ends where one wave per token no longer fits one block;
+// above, s is staged in k_rmsnorm and the dispatch alone takes about 4 us. tiles2: the
 // down GEMM's list, of at most NT2 tokens per tile (0: none).
 constexpr int ROUTE_SMALL_T = 8;
 __global__ void k_route_small(const float *logits, const float *bias, int has_bias, int K,

@@ -157,9 +157,6 @@ static int dalloc(P **p, size_t bytes) {
   return HY3X_OK;
 }
 
-// Up to this many tokens the router runs as one wave per (expert, token);
-// above it as RMSNorm + LDS-tiled GEMM + per-token top-K.
-constexpr int kSmallRouterT = 8;
 // From this many tokens the experts run as MFMA grouped GEMMs. Measured on MI355X the
 // MFMA tiles beat the wavefront-reduction GEMV tiles at every T >= 2 (T=2: 51 vs 66 us,
 // T=32: 442 vs 550 us for gate/up + down), so the GEMV tiles only run when selected
@@ -547,14 +544,16 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st, unsigned long
       // the routing kernels also clear (first kernel) and fill (top-K) the
       // dispatch bitmaps, or make the lists themselves (k_route_small); the
       // first kernel stages the MFMA operand
-      if (T <= kSmallRouterT) {
+      if (T <= ROUTE_SMALL_T) {
         const bool mf = c.mode == Mode::MFMA;
         k_router_logits<<<dim3(E, T), 256, 0, st>>>(x, c.xadd, L->norm_w, L->router, L->bias,
                                                     L->has_bias, S.logits, S.sig, S.score,
                                                     S.s16, S.s32, mf ? S.s16m : nullptr,
-                                                    S.ssum, L->trace[0], T,
-                                                    T <= ROUTE_SMALL_T ? nullptr : S.bits,
-                                                    S.wt, c.r_in);
+                                                    S.ssum, L->trace[0], c.r_in);
+        k_route_small<<<1, 64 * ROUTE_SMALL_T, 0, st>>>(
+            S.logits, L->bias, L->has_bias, K, c.scale, T, c.nt, S.ids, S.wpre, S.w, S.list,
+            S.tiles, S.n_tiles, mt, c.few ? FEW_TOKENS : 0, S.tiles2, S.n_tiles2, S.counts,
+            stats);
       } else {
         const bool mf = c.mode == Mode::MFMA;
         k_rmsnorm<<<T, 256, 0, st>>>(x, c.xadd, L->norm_w, mf ? nullptr : S.s16, S.s32,
@@ -568,13 +567,6 @@ static void launch_stage(hy3x_layer *L, int stage, hipStream_t st, unsigned long
   else
         HY3X_ROUTER_SHAPES(HY3X_LAUNCH_ROUTER) {}
 #undef HY3X_LAUNCH_ROUTER
-      }
-      if (T <= ROUTE_SMALL_T) {
-        k_route_small<<<1, 64 * ROUTE_SMALL_T, 0, st>>>(
-            S.logits, L->bias, L->has_bias, K, c.scale, T, c.nt, S.ids, S.wpre, S.w, S.list,
-            S.tiles, S.n_tiles, mt, c.few ? FEW_TOKENS : 0, S.tiles2, S.n_tiles2, S.counts,
-            stats);
-      } else {
         // one wave per token; up to 256 tokens one wave per block, so that
         // few tokens still spread over many CUs
         const int wpb = T <= 256 ? 1 : 4;

@@ -630,9 +630,11 @@ __global__ __launch_bounds__(MT_THREADS) void k_moe_mfma(
 template __global__ void k_moe_mfma<true>(const uint8_t *, const uint8_t *, const __half *,
                                           const __half *, const int32_t *, const int4 *,
                                           const int32_t *, int, int, __half *, float *);
+#ifndef HY3X_MFMA_TINY  // the 8-token shape runs gate/up only
 template __global__ void k_moe_mfma<false>(const uint8_t *, const uint8_t *, const __half *,
                                            const __half *, const int32_t *, const int4 *,
                                            const int32_t *, int, int, __half *, float *);
+#endif
 
 }  // namespace mfma_narrow / mfma_wide / mfma_tiny
 

@@ -35,9 +35,7 @@ __global__ __launch_bounds__(256) void k_router_logits(
     const float *__restrict__ router, const float *__restrict__ bias, int has_bias,
     float *__restrict__ logits, float *__restrict__ sig, float *__restrict__ score,
     __half *__restrict__ s16, float *__restrict__ s32, __half *__restrict__ s16m,
-    __half *__restrict__ ssum, unsigned long long *trace, int T,
-    uint32_t *__restrict__ bits, int wt, const float *__restrict__ r_in) {
-  if (bits) dispatch_clear_part(T, bits, wt, blockIdx.y * E + blockIdx.x, E * T);
+    __half *__restrict__ ssum, unsigned long long *trace, const float *__restrict__ r_in) {
   router_block(blockIdx.x, blockIdx.y, x, xadd, norm_w, router, bias, has_bias, logits, sig,
                score, s16, s32, s16m, ssum, trace, r_in);
 }
@@ -56,7 +54,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm(const float *__restrict__ x,
                                                  uint32_t *__restrict__ bits, int wt,
                                                  const float *__restrict__ r_in) {
   const int t = blockIdx.x, tid = threadIdx.x;
-  if (bits) dispatch_clear_part(T, bits, wt, t, T);
+  dispatch_clear_part(T, bits, wt, t, T);
   const float *xt = x + (size_t)t * D, *at = xadd ? xadd + (size_t)t * D : nullptr;
   const float4 *wg = reinterpret_cast<const float4 *>(norm_w);
   float4 a[4];
@@ -248,7 +246,7 @@ __global__ __launch_bounds__(256) void k_topk(const float *__restrict__ logits,
   const int t = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
   if (t >= T) return;  // whole waves
   const int my_e = route_token(logits, bias, has_bias, K, scale, t, ids, wpre, wout);
-  if (bits && lane < K) {
+  if (lane < K) {
     atomicOr(&bits[(size_t)my_e * wt + (t >> 5)], 1u << (t & 31));
     ranks[(size_t)my_e * wt * 32 + t] = (uint8_t)lane;  // lane k holds place k
   }
