@@ -17,8 +17,8 @@
 //    dmin and the mins are applied per block (see mfma_step).
 // All loads inside the column loop are these global->LDS copies, issued from
 // inline assembly: their completion is tracked by hand (s_waitcnt vmcnt on
-// the known number of copies in flight, then a barrier), which the compiler's
-// own wait insertion cannot do for LDS copies.
+// the known number of weight copies in flight, then a barrier), which the
+// compiler's own wait insertion cannot do for LDS copies.
 //
 // Operand layouts (16x16x32): lane l holds A[l%16][8(l/16) .. +7] (row, k),
 // B[8(l/16) .. +7][l%16] (k, column) and D[4(l/16) + i][l%16], i = 0..3. Here
@@ -177,9 +177,10 @@ __device__ __forceinline__ void apply_pending(TileState<GATEUP, NTT> &st) {
                                                st.acc[rg][m][t][i]);
 }
 
-// Copies of column kb: activations and sums into buffer kb & 1, then weights
-// of column ka into ring stage ka % 3 -- always B_DMA + 1 + A_DMA copies per
-// wave, weights last.
+// Copies of column kb: activations and sums into buffer kb & 1 (issue_b), weights
+// into ring stage kb % A_STAGES (issue_a). A wave issues A_DMA weight copies every
+// time, but only as many of its B_DMA + 1 others as the tile's tokens need, down to
+// none: a counted wait may count weight copies only.
 template <bool GATEUP, int NTT>
 __device__ __forceinline__ void issue_b(const TileState<GATEUP, NTT> &st, int kb) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -373,11 +374,12 @@ __device__ __forceinline__ void mfma_tile(const uint8_t *__restrict__ wq,
     st.aoff[j] = a_src<GATEUP>(wave, 64 * j + lane, rt, MAT_BYTES, NKB);
   st.a_last = 64 * (A_DMA - 1) + lane < A_CHUNKS_WAVE;
   // activations: copy j of wave w fills positions q = 64 (B_DMA w + j) + lane
-  // of the 32 x 32 chunk tile: row r = q / 32, position q % 32 holds chunk
+  // of the MT_TOK x 32 chunk tile: row r = q / 32, position q % 32 holds chunk
   // (q % 32) ^ (r & 15). Sums: lane (< S_LANES) of wave w fills position
-  // q = S_LANES w + lane of the 32 x 4 tile: row q / 4, position q % 4 holds
-  // part (q % 4) ^ ((row >> 2) & 3). Rows past n copy token 0's row (their D
-  // rows are never stored).
+  // q = S_LANES w + lane of the MT_TOK x 4 tile: row q / 4, position q % 4 holds
+  // part (q % 4) ^ ((row >> 2) & 3). Rows past n in the last copy that covers one
+  // of the tile's copy token 0's row, the rest is not copied (issue_b); their D
+  // rows are never stored.
   const int arow0 = t_arow[0];
   st.bbase = reinterpret_cast<const uint8_t *>(act);
   st.sbase = reinterpret_cast<const uint8_t *>(act_sum);
@@ -532,8 +534,8 @@ __device__ __forceinline__ void mfma_tile_q8(const uint8_t *__restrict__ wsh,
     st.aoff[j] = a_src<GATEUP>(wave, 64 * j + lane, rt, Q8_MAT_BYTES, NKB);
   st.a_last = 64 * (A_DMA - 1) + lane < A_CHUNKS_WAVE;
   // activations: copy j of wave w fills positions q = 64 (B8_DMA w + j) + lane
-  // of the 32 x 16 chunk tile: row r = q / 16, position q % 16 holds chunk
-  // (q % 16) ^ (r & 15). Rows past n copy token 0's row.
+  // of the MT_TOK x 16 chunk tile: row r = q / 16, position q % 16 holds chunk
+  // (q % 16) ^ (r & 15). Rows past n: as in mfma_tile.
   const int arow0 = t_arow[0];
   st.bbase = reinterpret_cast<const uint8_t *>(act);
 #pragma unroll
@@ -562,7 +564,7 @@ __device__ __forceinline__ void mfma_tile_q8(const uint8_t *__restrict__ wsh,
 // weights = gate and up rows of the expert (K = 4096), activations = staged
 // s, epilogue h = silu(g) * u -> h16m[slot][perm8(row)] (fp16). Otherwise
 // weights = down rows (K = 1536), activations = h16m, out[slot][row] fp32.
-// act_sum: sub-block sums of each activation row as (Sh, Sl, Sh, Sl) fp16.
+// act_sum: sub-block sums of each activation row, split (store_subsum).
 // wsh != nullptr: the shared expert's tiles use its Q8 matrices (mfma_tile_q8).
 template <bool GATEUP>
 __global__ __launch_bounds__(MT_THREADS) void k_moe_mfma(

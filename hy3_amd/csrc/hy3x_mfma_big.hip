@@ -91,8 +91,9 @@ __device__ __forceinline__ void set_weights(State<GATEUP, NTT> &st, const uint8_
   st.a_last = 64 * (A_DMA - 1) + lane < A_CHUNKS_WAVE;
 }
 
-// Copies (wave-uniform counts): weights A_DMA, activations X_DMA (those
-// covering rows past the tile's 16 NTT are skipped), sums S_DMA (idem).
+// Copies per wave: weights A_DMA every time, activations at most X_DMA and sums
+// at most S_DMA (those covering rows past the tile's 16 NTT are skipped): a counted
+// wait may count weight copies only.
 template <bool GATEUP, int NTT>
 __device__ __forceinline__ void issue_w(const State<GATEUP, NTT> &st, int kb) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -287,7 +288,8 @@ __device__ __forceinline__ void big_tile(const uint8_t *__restrict__ wq,
   // of the 128 x 16 half-column tile: row r = q / 16, position q % 16 holds
   // chunk (q % 16) ^ (r & 15) of the half. Sums: positions q = 64 (S_DMA w +
   // j) + lane of the 128 x 4 tile: row q / 4, position q % 4 holds part
-  // (q % 4) ^ ((row >> 2) & 3). Rows past n copy token 0's row.
+  // (q % 4) ^ ((row >> 2) & 3). Rows past n copy token 0's row, where a copy covers
+  // them.
   const int arow0 = t_arow[0];
   st.xbase = reinterpret_cast<const uint8_t *>(act);
   st.sbase = reinterpret_cast<const uint8_t *>(act_sum);

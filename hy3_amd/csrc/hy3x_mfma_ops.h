@@ -86,9 +86,11 @@ __device__ __forceinline__ void dequant_run(u2_t q, const PairScale &ps, h8_t &w
 // The mins operand of a row-block (header hd) for the lane's sub-blocks j = 2g
 // and 2g + 1 (their mins in the bytes of mw that sel picks): -dmin * m_j, each
 // split exactly into two fp16 parts hi + lo (dmin: 11 significant bits, m: 6;
-// the product's rounding error is one fused multiply-add away), against the
-// staged activation sums (Sh, Sl, Sh, Sl): the four cross products of the two
-// splits fill the MFMA's k slots. dmin is used as the half it is stored as:
+// the product's rounding error is one fused multiply-add away), laid out (hi, hi,
+// hi, hi, lo, lo, lo, lo) over the two sub-blocks in turn against the staged
+// activation sums (Sh, Sh, Sl, Sl, Sh, Sh, Sl, Sl: store_subsum): the four cross
+// products of the two splits fill the MFMA's k slots. dmin is used as the half it is
+// stored as:
 // hy3.c's decode (fp16_quirk) reads a half with exponent 0 as 2^-15 (1 + mant /
 // 1024), half of the half with exponent 1 and the same mantissa, so there m / 2
 // (exact) meets that one. In packed fp16 this takes nine vector instructions;
