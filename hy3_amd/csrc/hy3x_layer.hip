@@ -689,8 +689,14 @@ static int forward_impl(hy3x_layer *L, const Scratch *sc, const hy3x_layer **own
     return fail(HY3X_E_ARG, "T=%d outside [1,%d]", T, sc->max_tokens);
   if (K < 1 || K > KMAX) return fail(HY3X_E_ARG, "K=%d outside [1,8]", K);
   if (!L->router_set) return fail(HY3X_E_STATE, "router not set");
+  const Mode mode = T == 1 && L->path == 0                              ? Mode::DECODE
+                    : L->path >= 2 || (L->path == 0 && T >= kMfmaMinT) ? Mode::MFMA
+                                                                        : Mode::GEMV;
+  if (L->shared_q8 && mode == Mode::GEMV)
+    return fail(HY3X_E_STATE, "the GEMV tile path needs a Q4_K shared expert");
   hipStream_t st = (hipStream_t)stream;
-  auto &c = L->cur;
+  auto &c = L->cur;  // of the last forward until here: a refused call leaves it
+  c.mode = mode;
   c.x = x;
   c.xadd = xadd;
   c.T = T;
@@ -699,14 +705,6 @@ static int forward_impl(hy3x_layer *L, const Scratch *sc, const hy3x_layer **own
   c.sc = *sc;
   c.r_in = L->rms_n >= T ? L->rms_r : nullptr;
   L->rms_n = 0;  // a substituted scale serves one forward only
-  if (T == 1 && L->path == 0)
-    c.mode = Mode::DECODE;
-  else if (L->path >= 2 || (L->path == 0 && T >= kMfmaMinT))
-    c.mode = Mode::MFMA;
-  else
-    c.mode = Mode::GEMV;
-  if (L->shared_q8 && c.mode == Mode::GEMV)
-    return fail(HY3X_E_STATE, "the GEMV tile path needs a Q4_K shared expert");
   c.big = c.mode == Mode::MFMA &&
           (L->path == 5 || ((L->path == 0 || L->path == 2) && T >= kMfmaBigMinT));
   c.wide = c.mode == Mode::MFMA && !c.big &&

@@ -877,6 +877,23 @@ def test_q8_shared_keeps_narrow_gateup(torch, q8_layer, T, K):
     assert q8_layer.last_kernel("down") == "k_down_few"
 
 
+def test_refused_forward_leaves_the_last_one(torch, q8_layer):
+    """A forward refused for its path (GEMV tiles with the Q8_0 shared expert)
+    leaves what the layer says of its last forward: the routing, which the
+    refused static call would look for in another scratch, and the kernels."""
+    _, ids, wpre, _ = run(torch, q8_layer, C.inputs(0xCE, 4))
+    x = torch.zeros(3, D, device="cuda")
+    q8_layer.set_path(1)
+    try:
+        with pytest.raises(H.HY3XError, match="GEMV"):
+            q8_layer.forward_static(x.data_ptr(), 3, 2)
+    finally:
+        q8_layer.set_path(0)
+    assert q8_layer.last_kernel("down") == "k_down_few" and q8_layer.last_path() == 3
+    ids2, wpre2, _ = q8_layer.last_routing(4, 8)
+    assert np.array_equal(ids, ids2) and np.array_equal(wpre, wpre2)
+
+
 def test_q8_shared_reference_tokens(torch, q8_layer):
     """hy3.c's forward_layer_moe with the Q8_0 shared expert on three config-1
     tokens (moe_q8.npz), through the batched (MFMA) path."""
