@@ -58,10 +58,11 @@ __global__ void k_dispatch_list(const uint8_t *ranks, int T, int K, int NT, cons
 // Up to this many tokens the router runs as one wave per (expert, token)
 // (k_router_logits; above as RMSNorm + LDS-tiled GEMM + per-token top-K), and one
 // block routes every token and makes the dispatch lists (k_route_small), in one
-// launch where top-K, staging and dispatch were three: 2 / 3 / 4 / 8 tokens 73.4 / 99.5 / 108.0 / 155.9 -> 64.4 / 90.0 / 98.3 /
-// 145.9 us per forward. It ends where one wave per token no longer fits one block;
-// above, s is staged in k_rmsnorm and the dispatch alone takes about 4 us. tiles2: the
-// down GEMM's list, of at most NT2 tokens per tile (0: none).
+// launch where top-K, staging and dispatch were three: 2 / 3 / 4 / 8 tokens 73.4 /
+// 99.5 / 108.0 / 155.9 -> 64.4 / 90.0 / 98.3 / 145.9 us per forward. It ends where
+// one wave per token no longer fits one block; above, s is staged in k_rmsnorm and
+// the dispatch alone takes about 4 us. tiles2: the down GEMM's list, of at most NT2
+// tokens per tile (0: none).
 constexpr int ROUTE_SMALL_T = 8;
 __global__ void k_route_small(const float *logits, const float *bias, int has_bias, int K,
                               float scale, int T, int NT, int32_t *ids, float *wpre, float *wout,
@@ -160,7 +161,7 @@ extern template __global__ void k_moe_big<false>(const uint8_t *, const uint8_t 
 // The down GEMM for few tokens per expert (hy3x_mfma_few.hip): work tiles of
 // 16 FEW_WAVES rows and up to FEW_TOKENS tokens (up to FEW_ROWS: their h rows
 // whole in LDS).
-constexpr int FEW_TOKENS = 16, FEW_ROWS = 4, FEW_WAVES = 4;
+constexpr int FEW_TOKENS = 32, FEW_ROWS = 4, FEW_WAVES = 4;
 __global__ void k_down_few(const uint8_t *wq, const uint8_t *wsh, const __half *act,
                            const __half *act_sum, const int32_t *list, const int4 *tiles,
                            const int32_t *n_tiles, int T, float *out);

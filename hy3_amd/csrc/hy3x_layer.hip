@@ -175,13 +175,15 @@ constexpr int kMfmaMinT = 2;
 // launch, three to a CU later than two (K = 8, 3 tokens 49.6 vs 52.9, 4: 54.3 vs 56.3;
 // K = 4, 8: 51.8 vs 54.4).
 constexpr int kTinyMinRowTiles = 512, kTinyMaxRowTiles = 800;
-// Up to this many tokens the down GEMM keeps whole rows in registers (k_down_few):
-// three tiles of 16 tokens of an expert at most. Down launch us, K = 8, weights from
-// HBM, narrow tiles vs whole rows, tokens evenly spread: 2 tokens 21.7 vs 18.9, 8:
-// 48.5 vs 39.7, 32: 94.5 vs 81.9, 48: 107.6 vs 97.1, 64: 115.5 vs 109.0, 96: 126.9 vs
-// 124.2; every token on the same eight experts: 8: 15.3 vs 15.4, 32: 19.0 vs 20.6, 48:
-// 22.2 vs 26.0, but 56: 24.5 vs 30.4, 64: 24.8 vs 30.6. The dispatch is not known
-// on the host, so the line lies where a fourth tile would begin.
+// Up to this many tokens the down GEMM keeps whole rows in registers (k_down_few). The
+// dispatch is not known on the host, so the line lies where what it gains on spread
+// tokens no longer outweighs what it loses where every token chooses the same eight
+// experts. Down launch us, K = 8, three layers in rotation, narrow tiles vs whole rows,
+// evenly spread: 2 tokens 20.4 vs 16.1, 8: 47.5 vs 38.0, 32: 93.3 vs 79.3, 48: 105.7 vs
+// 96.5, 64: 117.7 vs 109.8, 96: 126.1 vs 123.5; a few popular experts: 48: 127.7 vs
+// 109.6; the same eight: 8: 14.4 vs 14.6, 32: 17.0 vs 17.8, 48: 21.3 vs 21.4, 64: 24.6 vs
+// 25.0, 96: 30.2 vs 31.8. Whole forwards at 48 tokens -2.5 %, -4.3 % and +0.7 % at worst
+// (Q8 shared expert -2.4, -4.2 and +3.3), at 96 0, -2.4 and +2.5 (0, -1.9 and +5.2).
 constexpr int kDownFewMaxT = 48;
 // From this many tokens the MFMA GEMMs use the wide tile shape (64 tokens, 8 waves).
 // Measured on MI355X (ms per layer, narrow vs wide): 32 tokens 0.32 vs 0.37,

@@ -1,5 +1,5 @@
 // hy3x_mfma_few.hip -- the grouped down GEMM for few tokens per expert: a wave's
-// whole weight rows in registers, no barrier in the reduction.
+// whole weight rows in registers.
 //
 // With few tokens per expert the down GEMM is bound by how the weights stream:
 // the narrow MFMA tiles (hy3x_mfma.hip) walk 128-row tiles column by column, 144
@@ -9,20 +9,23 @@
 // its registers (72 VGPRs per lane; every 128-byte line is requested once and
 // used whole). A workgroup is four such waves, four workgroups per CU.
 //
-// A work tile has up to FEW_TOKENS = 16 tokens, one MFMA row group, so an expert
-// with n tokens has its rows read and dequantised ceil(n / 16) times. Up to
-// FEW_ROWS = 4 tokens the tokens' h rows are staged in LDS whole and the reduction
-// has no barrier; above, whole rows would leave no room for four workgroups, and
-// they are staged a column at a time. (All tiles of up to 4 tokens: every token on
-// the same eight experts 25.1 / 42.7 / 59.0 us at 16 / 32 / 48 tokens, 16.6 / 20.6 /
-// 26.0 now, the narrow tiles 16.3 / 19.0 / 22.2; all of up to 8, rows whole: evenly
-// spread 42 and 65 us at 8 and 16.)
+// A work tile has up to FEW_TOKENS = 32 tokens, two MFMA row groups, so an expert with
+// n tokens has its rows read and dequantised ceil(n / 32) times. Up to FEW_ROWS = 4
+// tokens the tokens' h rows are staged in LDS whole and the reduction has no barrier;
+// above, whole rows would leave no room for four workgroups, and they are staged a
+// column at a time. Down launch where every token chooses the same eight experts, at
+// 16 / 24 / 32 / 48 tokens: narrow tiles 14.9 / 16.4 / 17.0 / 21.3 us, here 15.1 / 17.3 /
+// 17.8 / 21.4; with tiles of up to 16 tokens 14.7 / 18.6 / 18.9 / 22.8; of up to 4 about
+// 1.5 to 2.6 times the narrow tiles'. (All of up to 8, rows whole: evenly spread 42 and
+// 65 us at 8 and 16.) With a Q8 shared expert there 17.8 and 20.8 us at 32 and 40, here
+// 20.3 and 21.6 (tiles of 16: 20.6 and 25.8): a Q8 row does not fit the registers.
 //
 // Down launch, weights from HBM, evenly spread over the experts, narrow tiles and
-// here: 3 tokens 27.3 and 22.7 us, 8: 48.5 and 39.7, 16: 71.6 and 58.4, 32: 94.5 and
-// 81.9, 48: 107.6 and 97.1. Measured beside it: the columns one, two or three at a
+// here: 3 tokens 24.8 and 19.6 us, 8: 47.5 and 38.0, 16: 72.2 and 57.6, 32: 93.3 and
+// 79.3, 48: 105.7 and 96.5. Measured beside it: the columns one, two or three at a
 // time through a register ring slower than the narrow tiles at 8 tokens, two or
-// eight waves per workgroup 2-8 % slower.
+// eight waves per workgroup 2-8 % slower, three column pairs of a Q8 row in flight
+// instead of two spill.
 //
 // The arithmetic per element is the MFMA tiles': the same operands, k order and
 // sequence of operations on every accumulator (hy3x_mfma.hip's header), so a
@@ -41,11 +44,12 @@ constexpr int FW_SC = F / 32 * 8 / 16;         // and of its sums (24)
 constexpr int FW_XROW = FW_XC + 4, FW_SROW = FW_SC + 4;  // LDS row strides, whole rows
 constexpr int FW_CXC = FW_XC / FW_NKB, FW_CSC = FW_SC / FW_NKB;  // chunks of one column (32, 4)
 constexpr int FW_CXROW = FW_CXC + 1, FW_CSROW = FW_CSC + 1;      // LDS row strides, one column
-constexpr int FW_COL = FEW_TOKENS * (FW_CXROW + FW_CSROW);       // one column of a tile in LDS
+constexpr int FW_COL = 16 * (FW_CXROW + FW_CSROW);  // one column of a row group in LDS
+constexpr int FW_GROUPS = FEW_TOKENS / 16;          // MFMA row groups of a tile
 constexpr int FW_THREADS = 64 * FEW_WAVES;
-constexpr int FW_LDS = FEW_ROWS * (FW_XROW + FW_SROW) > 2 * FW_COL
-                           ? FEW_ROWS * (FW_XROW + FW_SROW) : 2 * FW_COL;
-static_assert(FEW_TOKENS == 16 && (FEW_ROWS & (FEW_ROWS - 1)) == 0, "one MFMA row group");
+constexpr int FW_LDS = 2 * FW_GROUPS * FW_COL;
+static_assert(FW_GROUPS == 2 && FEW_ROWS <= 16 && (FEW_ROWS & (FEW_ROWS - 1)) == 0, "row groups");
+static_assert(FEW_ROWS * (FW_XROW + FW_SROW) <= FW_LDS, "whole rows");
 
 // A lane's part of its whole down row in Q4_K.
 struct FewRow {
@@ -59,12 +63,18 @@ struct FewRow {
       q[kb][1] = p[5 + g];
     }
   }
-  // column kb: xc its 32 chunks of this lane's MFMA row, sv the lane's sums
-  __device__ __forceinline__ f4_t column(int kb, const u4_t *xc, u4_t sv, int g, f4_t acc) const {
+  // column kb of NG row groups, each dequantised weight used for all of them: xc its
+  // 32 chunks of this lane's MFMA row and sc the lane's sums, xs and ss from one
+  // group's to the next's
+  template <int NG>
+  __device__ __forceinline__ void column(int kb, const u4_t *xc, int xs, const u4_t *sc, int ss,
+                                         int g, f4_t (&acc)[NG]) const {
     const uint32_t sel = bytes_sel(g >> 1), msel = bytes_sel(g & 1);
     const int gch = 8 * (g >> 1) + 2 * (g & 1);
     const Scales6 s6 = unpack_scales(hdr[kb]);
-    f4_t dblk = {0.f, 0.f, 0.f, 0.f};
+    f4_t dblk[NG];
+#pragma unroll
+    for (int r = 0; r < NG; r++) dblk[r] = (f4_t){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int piece = 0; piece < 2; piece++) {
       const PairScale ps = pair_scale(s6.sc[piece], sel);
@@ -73,16 +83,22 @@ struct FewRow {
       dequant_run(q[kb][piece].zw, ps, wf[1], wf[3]);
 #pragma unroll
       for (int hu = 0; hu < 4; hu++)
-        dblk = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-            __builtin_bit_cast(h8_t, xc[16 * piece + 4 * (hu >> 1) + (hu & 1) + gch]), wf[hu],
-            dblk, 0, 0, 0);
+#pragma unroll
+        for (int r = 0; r < NG; r++)
+          dblk[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              __builtin_bit_cast(h8_t,
+                                 xc[r * xs + 16 * piece + 4 * (hu >> 1) + (hu & 1) + gch]),
+              wf[hu], dblk[r], 0, 0, 0);
     }
     const h8_t mo = mins_operand(hdr[kb].x, (g >> 1) ? s6.mn[1] : s6.mn[0], msel);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, sv), mo, acc, 0, 0, 0);
     const float d = fp16_quirk(hdr[kb].x & 0xffffu);
 #pragma unroll
-    for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(d, dblk[i], acc[i]);
-    return acc;
+    for (int r = 0; r < NG; r++) {
+      acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(h8_t, sc[r * ss]), mo,
+                                                      acc[r], 0, 0, 0);
+#pragma unroll
+      for (int i = 0; i < 4; i++) acc[r][i] = __builtin_fmaf(d, dblk[r][i], acc[r][i]);
+    }
   }
 };
 
@@ -95,63 +111,92 @@ struct FewQ8 {
 #pragma unroll
     for (int b = 0; b < 4; b++) q[b] = *reinterpret_cast<const u2_t *>(p + 16 + 32 * b + 8 * g);
   }
-  // xc: the column's 16 chunks of this lane's MFMA row
-  __device__ __forceinline__ f4_t column(const u4_t *xc, int g, f4_t acc) const {
+  // xc: the column's 16 chunks of this lane's MFMA row, xs from one group's to the next's
+  template <int NG>
+  __device__ __forceinline__ void column(const u4_t *xc, int xs, int g, f4_t (&acc)[NG]) const {
     const f4_t zero4 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int b = 0; b < 4; b++) {
-      const f4_t pr = __builtin_amdgcn_mfma_f32_16x16x32_f16(
-          __builtin_bit_cast(h8_t, xc[4 * b + g]), q8_run(q[b]), zero4, 0, 0, 0);
+      const h8_t wf = q8_run(q[b]);
 #pragma unroll
-      for (int i = 0; i < 4; i++) acc[i] = __builtin_fmaf(dsc[b], pr[i], acc[i]);
+      for (int r = 0; r < NG; r++) {
+        const f4_t pr = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+            __builtin_bit_cast(h8_t, xc[r * xs + 4 * b + g]), wf, zero4, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; i++) acc[r][i] = __builtin_fmaf(dsc[b], pr[i], acc[r][i]);
+      }
     }
-    return acc;
   }
 };
 
-// A tile of more than FEW_ROWS tokens: its rows would not fit LDS whole beside
-// three other workgroups, so they are staged a column at a time (two buffers, a
-// third column in registers), 16 threads per token; tokens past the tile's repeat
-// its last. The weights are requested after those and stay whole in registers.
-template <bool Q8>
-__device__ __forceinline__ f4_t few_tile_columns(const uint8_t *wrow, const __half *act,
+// acc of row group r: lane holds D[token 16 r + 4g + i][its row].
+__device__ __forceinline__ void few_store(const f4_t &acc, int r, const int32_t *slots, int n,
+                                          int g, int row, float *out) {
+#pragma unroll
+  for (int i = 0; i < 4; i++)
+    if (16 * r + 4 * g + i < n) out[(size_t)slots[16 * r + 4 * g + i] * D + row] = acc[i];
+}
+
+// A tile of more than FEW_ROWS tokens, in NG row groups: its rows would not fit LDS
+// whole beside three other workgroups, so they are staged a column at a time (two
+// buffers, a third column in registers), 16 threads per token of a group; tokens past
+// the tile's repeat its last. The weights are requested after those and stay whole in
+// registers.
+template <bool Q8, int NG>
+__device__ __forceinline__ void few_tile_columns(const uint8_t *wrow, const __half *act,
                                                  const __half *act_sum, const int32_t *slots,
-                                                 int n, u4_t *lds) {
+                                                 int n, int row, float *out, u4_t *lds) {
+  constexpr int COL = NG * FW_COL, XG = 16 * FW_CXROW, SG = 16 * FW_CSROW;
   const int tid = threadIdx.x, lr = tid & 15, g = (tid >> 4) & 3;
-  const int t = tid >> 4, c = tid & 15, cs = c & (FW_CSC - 1);
-  static_assert(FW_THREADS == 16 * FEW_TOKENS && FW_CXC == 32 && FW_CSC == 4, "staging split");
+  // the thread's chunks c and c + 16 of token t of every group, and part cs of the sums
+  // of token ts (four lanes hold the same, or two of either group)
+  const int t = tid >> 4, c = tid & 15, cs = c & (FW_CSC - 1), ts = t + 16 * ((c >> 2) % NG);
+  static_assert(FW_THREADS == 16 * 16 && FW_CXC == 32 && FW_CSC == 4 && NG <= 2, "staging split");
   struct Col {
-    u4_t x[2], s;
+    u4_t x[NG][2], s;
   };
-  const int slot = slots[min(t, n - 1)];
-  const char *xs = reinterpret_cast<const char *>(act) + (uint32_t)(slot * (F * 2) + 16 * c);
-  const char *ss =
-      reinterpret_cast<const char *>(act_sum) + (uint32_t)(slot * (F / 32 * 8) + 16 * cs);
+  const char *ab = reinterpret_cast<const char *>(act);
+  const char *sb = reinterpret_cast<const char *>(act_sum);
+  uint32_t xo[NG];
+#pragma unroll
+  for (int r = 0; r < NG; r++)
+    xo[r] = (uint32_t)(slots[min(16 * r + t, n - 1)] * (F * 2) + 16 * c);
+  const uint32_t so = (uint32_t)(slots[min(ts, n - 1)] * (F / 32 * 8) + 16 * cs);
   auto request = [&](int kb) {
     Col o;
-    o.x[0] = *reinterpret_cast<const u4_t *>(xs + kb * (16 * FW_CXC));
-    o.x[1] = *reinterpret_cast<const u4_t *>(xs + kb * (16 * FW_CXC) + 256);
-    if (!Q8) o.s = *reinterpret_cast<const u4_t *>(ss + kb * (16 * FW_CSC));
+#pragma unroll
+    for (int r = 0; r < NG; r++) {
+      o.x[r][0] = *reinterpret_cast<const u4_t *>(ab + (xo[r] + kb * (16 * FW_CXC)));
+      o.x[r][1] = *reinterpret_cast<const u4_t *>(ab + (xo[r] + kb * (16 * FW_CXC) + 256));
+    }
+    if (!Q8) o.s = *reinterpret_cast<const u4_t *>(sb + (so + kb * (16 * FW_CSC)));
     return o;
   };
   auto stage = [&](int kb, const Col &o) {
-    u4_t *b = lds + (kb & 1) * FW_COL;
-    b[t * FW_CXROW + c] = o.x[0];
-    b[t * FW_CXROW + c + 16] = o.x[1];
-    if (!Q8) b[FEW_TOKENS * FW_CXROW + t * FW_CSROW + cs] = o.s;  // four lanes, the same value
+    u4_t *b = lds + (kb & 1) * COL;
+#pragma unroll
+    for (int r = 0; r < NG; r++) {
+      b[r * XG + t * FW_CXROW + c] = o.x[r][0];
+      b[r * XG + t * FW_CXROW + c + 16] = o.x[r][1];
+    }
+    if (!Q8) b[NG * XG + ts * FW_CSROW + cs] = o.s;
   };
   const Col c0 = request(0), c1 = request(1);
-  Col next = request(2);
+  Col next;
   auto stage_first = [&] {
     __builtin_amdgcn_sched_barrier(0);
     stage(0, c0);
     stage(1, c1);
     __syncthreads();
   };
-  f4_t acc = {0.f, 0.f, 0.f, 0.f};
-  // After column kb: once every wave has read its buffer, kb + 2 goes there (read after
-  // the barrier of kb + 1). The last two columns stage one more, which nothing reads.
+  f4_t acc[NG];
+#pragma unroll
+  for (int r = 0; r < NG; r++) acc[r] = (f4_t){0.f, 0.f, 0.f, 0.f};
   if constexpr (Q8) {
+    // After column kb: once every wave has read its buffer, kb + 2 goes there (read
+    // after the barrier of kb + 1). The last two columns stage one more, which nothing
+    // reads.
+    next = request(2);
     constexpr int QD = 2;  // column pairs (256 of K) in flight
     static_assert(FW_NKB % QD == 0, "whole rounds of the ring");
     FewQ8 w[QD][2];
@@ -167,9 +212,9 @@ __device__ __forceinline__ f4_t few_tile_columns(const uint8_t *wrow, const __ha
 #pragma unroll
       for (int i = 0; i < QD; i++) {
         const int kb = k0 + i;
-        const u4_t *xc = lds + (kb & 1) * FW_COL + lr * FW_CXROW;
+        const u4_t *xc = lds + (kb & 1) * COL + lr * FW_CXROW;
 #pragma unroll
-        for (int j = 0; j < 2; j++) acc = w[i][j].column(xc + 16 * j, g, acc);
+        for (int j = 0; j < 2; j++) w[i][j].column(xc + 16 * j, XG, g, acc);
         request_w(min(kb + QD, FW_NKB - 1), w[i]);
         __syncthreads();
         stage(kb, next);
@@ -181,21 +226,24 @@ __device__ __forceinline__ f4_t few_tile_columns(const uint8_t *wrow, const __ha
     stage_first();
 #pragma unroll
     for (int kb = 0; kb < FW_NKB; kb++) {
-      const u4_t *b = lds + (kb & 1) * FW_COL;
-      acc = w.column(kb, b + lr * FW_CXROW, b[FEW_TOKENS * FW_CXROW + lr * FW_CSROW + g], g, acc);
+      const u4_t *b = lds + (kb & 1) * COL;
+      w.column(kb, b + lr * FW_CXROW, XG, b + NG * XG + lr * FW_CSROW + g, SG, g, acc);
+      // column kb + 1 goes to the buffer that every wave had read at the last barrier;
+      // kb + 2 is requested as late as that, when column kb's weights have made room
+      if (kb >= 1 && kb + 1 < FW_NKB) stage(kb + 1, next);
       if (kb + 1 < FW_NKB) __syncthreads();
-      if (kb + 2 < FW_NKB) stage(kb, next);
-      if (kb + 3 < FW_NKB) next = request(kb + 3);
+      if (kb + 2 < FW_NKB) next = request(kb + 2);
     }
   }
-  return acc;
+#pragma unroll
+  for (int r = 0; r < NG; r++) few_store(acc[r], r, slots, n, g, row, out);
 }
 
 // A tile of at most FEW_ROWS tokens: its rows in LDS whole, one barrier.
 template <bool Q8>
-__device__ __forceinline__ f4_t few_tile_rows(const uint8_t *wrow, const __half *act,
+__device__ __forceinline__ void few_tile_rows(const uint8_t *wrow, const __half *act,
                                               const __half *act_sum, const int32_t *slots, int n,
-                                              u4_t *lds) {
+                                              int row, float *out, u4_t *lds) {
   const int tid = threadIdx.x, lr = tid & 15, g = (tid >> 4) & 3;
   u4_t *x_l = lds, *s_l = lds + FEW_ROWS * FW_XROW;
   // staging: 64 threads per token. Every row is written (zeros past the tile's
@@ -225,14 +273,14 @@ __device__ __forceinline__ f4_t few_tile_rows(const uint8_t *wrow, const __half 
   };
   const u4_t *xr = x_l + (lr & (FEW_ROWS - 1)) * FW_XROW;
   const u4_t *sr = s_l + (lr & (FEW_ROWS - 1)) * FW_SROW;
-  f4_t acc = {0.f, 0.f, 0.f, 0.f};
+  f4_t acc[1] = {{0.f, 0.f, 0.f, 0.f}};
   if constexpr (Q8) {  // 128 of K per 144-byte column
     stage();
 #pragma unroll 4
     for (int kb = 0; kb < F / Q8K; kb++) {
       FewQ8 w8;
       w8.request(wrow + (size_t)kb * QB, g);
-      acc = w8.column(xr + 16 * kb, g, acc);
+      w8.column(xr + 16 * kb, 0, g, acc);
     }
   } else {
     // the rows were requested before the weights (loads complete in the order they
@@ -244,9 +292,9 @@ __device__ __forceinline__ f4_t few_tile_rows(const uint8_t *wrow, const __half 
     stage();
 #pragma unroll
     for (int kb = 0; kb < FW_NKB; kb++)
-      acc = w.column(kb, xr + FW_CXC * kb, sr[FW_CSC * kb + g], g, acc);
+      w.column(kb, xr + FW_CXC * kb, 0, sr + FW_CSC * kb + g, 0, g, acc);
   }
-  return acc;
+  few_store(acc[0], 0, slots, n, g, row, out);
 }
 
 __global__ __launch_bounds__(FW_THREADS, 4) void k_down_few(
@@ -261,24 +309,28 @@ __global__ __launch_bounds__(FW_THREADS, 4) void k_down_few(
   const int w = xcd_remap(blockIdx.x, nreal, (T + FEW_TOKENS - 1) / FEW_TOKENS * NRT);
   const int4 td = tiles[w / NRT];
   const int e = td.x, n = td.z;
-  const int tid = threadIdx.x, lr = tid & 15, g = (tid >> 4) & 3;
+  const int tid = threadIdx.x, lr = tid & 15;
   const bool q8 = wsh != nullptr && e == E;
   const int row = w % NRT * TROWS + 16 * (tid >> 6) + lr;
   const uint8_t *wrow = q8 ? wsh + 2 * Q8_MAT_BYTES + (size_t)row * (F / Q8K) * QB
                            : wq + (size_t)e * EXPERT_BYTES + 2 * MAT_BYTES +
                                  (size_t)row * FW_NKB * QB;
   const int32_t *slots = list + td.y;
-  f4_t acc;
-  if (n <= FEW_ROWS)
-    acc = q8 ? few_tile_rows<true>(wrow, act, act_sum, slots, n, lds)
-             : few_tile_rows<false>(wrow, act, act_sum, slots, n, lds);
-  else
-    acc = q8 ? few_tile_columns<true>(wrow, act, act_sum, slots, n, lds)
-             : few_tile_columns<false>(wrow, act, act_sum, slots, n, lds);
-  // lane holds D[token 4g + i][its row]
-#pragma unroll
-  for (int i = 0; i < 4; i++)
-    if (4 * g + i < n) out[(size_t)slots[4 * g + i] * D + row] = acc[i];
+  if (n <= FEW_ROWS) {
+    if (q8)
+      few_tile_rows<true>(wrow, act, act_sum, slots, n, row, out, lds);
+    else
+      few_tile_rows<false>(wrow, act, act_sum, slots, n, row, out, lds);
+  } else if (n <= 16) {
+    if (q8)
+      few_tile_columns<true, 1>(wrow, act, act_sum, slots, n, row, out, lds);
+    else
+      few_tile_columns<false, 1>(wrow, act, act_sum, slots, n, row, out, lds);
+  } else if (q8) {
+    few_tile_columns<true, 2>(wrow, act, act_sum, slots, n, row, out, lds);
+  } else {
+    few_tile_columns<false, 2>(wrow, act, act_sum, slots, n, row, out, lds);
+  }
 }
 
 }  // namespace hy3x
